@@ -372,7 +372,7 @@ int rdhip_evolve_bwd(rdhip_ctx* ctx, const void* grad_chosen, void* grad_points,
  * choose of rdhip_choose (rd/cpu/brute_force/choose.hpp:36-70) on caller-owned device buffers,
  * with no context.  It allocates nothing, copies nothing and does not synchronise: it only
  * enqueues kernels on hip_stream (NULL = the null stream), which must belong to the current
- * device.  Its work memory (about 16 MiB) is a fixed device array of the library, one per
+ * device.  Its work memory (about 2 MiB) is a fixed device array of the library, one per
  * device, held until the process ends; calls that overlap on one device race.
  *   points:  n points (device), COL_MAJOR / SOA: coordinate d of point i at points[d*stride + i]
  *            (stride >= n, 0 = n); n in [1, RDHIP_NOALLOC_MAX_POINTS];

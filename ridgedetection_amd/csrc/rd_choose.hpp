@@ -16,14 +16,24 @@ struct ChooseArgs {
     int numSegs;
     int* segK;
     const T* segRSqr;
-    unsigned char* covered;   // per sample: covered by the chosen set at its chunk's start
     int* chosenIdx;           // per chosen slot: segment-relative index of the chosen sample
     int* overflow;
-    const int* segLarge;      // per segment: 1 = chunked path (filter + block), 0 = one block
+    // large segments (rounds of resolve and filter); small ones run in one block each
+    const int* segLarge;      // per segment: 1 = large
+    int numLarge;
+    const int* largeSeg;      // [numLarge] their indices
+    const int* largeBlock;    // [numLarge + 1] first filter block of each (kChooseBlock samples a block)
+    uint64_t* open;           // one bit per own sample, 4 words per filter block; set: not decided yet
+    int* base;                // [numLarge] chosen points the open samples have been tested against
+    int* cursor;              // [numLarge] first word of the segment that may hold an open sample
+    int* doneCount;           // large segments without an open sample
 };
 
-// Chunk schedule of the large-segment path: chunk c covers samples
-// [choose_chunk_start(c), choose_chunk_start(c+1)).  Chunk 0 is the sequential start.
+constexpr int kChooseBlock = 256;    // samples per filter block: one word of `open` per wave
+constexpr int kChooseBatch = 1024;   // candidates one resolve step decides
+
+// Chunk schedule of the fixed-launch form (rdhip_choose_noalloc): chunk c covers samples
+// [choose_chunk_start(c), choose_chunk_start(c+1)).
 __host__ __device__ inline int choose_chunk_start(int c) {
     if (c <= 0) return 0;
     if (c == 1) return 2048;
@@ -33,10 +43,20 @@ __host__ __device__ inline int choose_chunk_start(int c) {
     return v > 0x7fffffffLL ? 0x7fffffff : (int)v;
 }
 
+// every small segment, one block each
 template <typename T>
-hipError_t launch_choose_filter(const ChooseArgs<T>& a, int dim, const WorkItem* items, int numItems,
+hipError_t launch_choose_small(const ChooseArgs<T>& a, int dim, hipStream_t st);
+// all samples of the large segments open, nothing chosen
+template <typename T>
+hipError_t launch_choose_open(const ChooseArgs<T>& a, int numBlocks, hipStream_t st);
+// tests the open samples of filter blocks [block0, block0 + numBlocks) against the chosen points
+// added since the last test (fresh: every sample of the blocks against all chosen points)
+template <typename T>
+hipError_t launch_choose_filter(const ChooseArgs<T>& a, int dim, int block0, int numBlocks, bool fresh,
                                 hipStream_t st);
+// decides the first open samples of every large segment: up to maxBatches batches of
+// kChooseBatch (0: all of them), of the samples below endSample only (< 0: all)
 template <typename T>
-hipError_t launch_choose_block(const ChooseArgs<T>& a, int dim, int chunk, int useFlags, hipStream_t st);
+hipError_t launch_choose_resolve(const ChooseArgs<T>& a, int dim, int endSample, int maxBatches, hipStream_t st);
 
 }  // namespace rdhip

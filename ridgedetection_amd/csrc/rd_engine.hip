@@ -19,6 +19,10 @@ namespace rdhip {
 
 namespace {
 
+constexpr int kChooseFewSegs = 256;        // one block per CU
+constexpr int kChooseLargeFew = 4096;
+constexpr int kChooseLargeMany = 32768;
+
 inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
 __global__ void fill_int_kernel(int* __restrict__ a, int64_t n, int v, const int* __restrict__ skip) {
@@ -125,7 +129,6 @@ Engine<T>::~Engine() {
     if (decWs_.nbr) (void)hipFree(decWs_.nbr);
     if (decWs_.par) (void)hipFree(decWs_.par);
     if (decWs_.boxes) (void)hipFree(decWs_.boxes);
-    for (auto* b : chooseItems_) delete b;
 }
 
 template <typename T>
@@ -283,9 +286,6 @@ void Engine<T>::buildWorkItems() {
     if (!items.empty())
         check(hipMemcpyAsync(dItems_.get(), items.data(), sizeof(WorkItem) * items.size(), hipMemcpyHostToDevice, st_),
               "items");
-    // choose filter items for the chunked (large segment) path
-    for (auto* b : chooseItems_) delete b;
-    chooseItems_.clear();
 }
 
 // Longest-first order for the persistent scan's work queue: cost ~ samples x live chosen.
@@ -405,7 +405,6 @@ void Engine<T>::ensureEvolveScratch() {
         cKeys_.reserve(totalP);
         cPos_.reserve(totalP);
     }
-    covered_.reserve(totalP);
     const int64_t slots = std::max<int64_t>(totalSlots_, 1);
     chainOff_.reserve(slots);
     chainEnd_.reserve(slots);
@@ -590,51 +589,56 @@ void Engine<T>::choose() {
     ++version_;
     chosenFromPoints_ = true;
     auto t0 = std::chrono::steady_clock::now();
-    constexpr int kLarge = 32768;
-    std::vector<int> large(ns);
-    int maxOwn = 0;
-    bool anyLarge = false;
+    // Large segments take the rounds of rd_choose.hip, the others one block each.  One block
+    // decides about 20 batches of 1024 samples in the time of one round's two launches and its
+    // share of the read-back, so a lone cloud gains from a few thousand samples on; hundreds of
+    // segments fill the GPU with a block each, and only ones too long for a block leave it.
+    const int largeMin = ns <= kChooseFewSegs ? kChooseLargeFew : kChooseLargeMany;
+    std::vector<int> info((size_t)ns), ids, first;
+    int blocks = 0;
     for (int s = 0; s < ns; ++s) {
-        large[s] = segs_[s].nOwn > kLarge ? 1 : 0;
-        anyLarge |= large[s] != 0;
-        if (large[s]) maxOwn = std::max(maxOwn, segs_[s].nOwn);
+        info[s] = segs_[s].nOwn > largeMin ? 1 : 0;
+        if (!info[s]) continue;
+        ids.push_back(s);
+        first.push_back(blocks);
+        blocks += (segs_[s].nOwn + kChooseBlock - 1) / kChooseBlock;
     }
-    DevBuf<int> dLarge;
-    dLarge.reserve(ns);
-    check(hipMemcpyAsync(dLarge.get(), large.data(), sizeof(int) * ns, hipMemcpyHostToDevice, st_), "large");
-    int zero = 0;
-    check(hipMemcpyAsync(flags_.get() + 2, &zero, sizeof(int), hipMemcpyHostToDevice, st_), "overflow");
+    const int nL = (int)ids.size();
+    first.push_back(blocks);
+    info.insert(info.end(), ids.begin(), ids.end());
+    info.insert(info.end(), first.begin(), first.end());
+    const size_t status = info.size();
+    info.insert(info.end(), 2, 0);   // overflow flag, finished large segments
+    chooseInfo_.reserve(info.size() + 2 * (size_t)nL);
+    chooseOpen_.reserve((size_t)blocks * (kChooseBlock / kWave));
+    check(hipMemcpyAsync(chooseInfo_.get(), info.data(), sizeof(int) * info.size(), hipMemcpyHostToDevice, st_),
+          "choose segments");
+    int* ci = chooseInfo_.get();
     ChooseArgs<T> a{es.P, es.stride, es.index, S_.get(), sStride_, dSegs_.get(), ns, dSegK_.get(), dSegR1Sqr_.get(),
-                    covered_.get(), chosenIdx_.get(), flags_.get() + 2, dLarge.get()};
-    // small segments: one block each, whole segment
-    check(launch_choose_block<T>(a, dim_, -1, 0, st_), "choose_block");
-    if (anyLarge) {
-        // chunk 0 sequentially, then filter + resolve per chunk
-        check(launch_choose_block<T>(a, dim_, 0, 0, st_), "choose_block");
-        std::vector<DevBuf<WorkItem>> bufs;
-        for (int c = 1; choose_chunk_start(c) < maxOwn; ++c) {
-            std::vector<WorkItem> items;
-            const int c0 = choose_chunk_start(c), c1 = choose_chunk_start(c + 1);
-            for (int s = 0; s < ns; ++s) {
-                if (!large[s]) continue;
-                const int e = std::min(c1, segs_[s].nOwn);
-                for (int st = c0; st < e; st += 1024) items.push_back({s, st, std::min(e, st + 1024), 0});
+                    chosenIdx_.get(), ci + status, ci, nL, ci + ns, ci + ns + nL, chooseOpen_.get(),
+                    ci + status + 2, ci + status + 2 + nL, ci + status + 1};
+    int got[2] = {0, 0};
+    if (nL < ns) check(launch_choose_small<T>(a, dim_, st_), "choose_small");
+    if (nL > 0) {
+        check(launch_choose_open<T>(a, blocks, st_), "choose_open");
+        check(launch_choose_resolve<T>(a, dim_, -1, 1, st_), "choose_resolve");
+        // a cloud whose samples are covered by a few hundred points is done after a handful of
+        // rounds; every read-back costs about as much as two of them
+        for (int rounds = 4; got[1] < nL; rounds = std::min(2 * rounds, 64)) {
+            for (int r = 0; r < rounds; ++r) {
+                check(launch_choose_filter<T>(a, dim_, 0, blocks, false, st_), "choose_filter");
+                check(launch_choose_resolve<T>(a, dim_, -1, 1, st_), "choose_resolve");
             }
-            if (items.empty()) continue;
-            DevBuf<WorkItem> buf;
-            buf.reserve(items.size());
-            check(hipMemcpyAsync(buf.get(), items.data(), sizeof(WorkItem) * items.size(), hipMemcpyHostToDevice, st_),
-                  "items");
-            check(launch_choose_filter<T>(a, dim_, buf.get(), (int)items.size(), st_), "choose_filter");
-            check(launch_choose_block<T>(a, dim_, c, 1, st_), "choose_block");
-            check(hipStreamSynchronize(st_), "choose chunk");
+            check(hipMemcpyAsync(got, ci + status, sizeof(got), hipMemcpyDeviceToHost, st_), "choose status");
+            check(hipStreamSynchronize(st_), "choose");
         }
     }
     fillSentinels();
-    int ovf = 0;
-    check(hipMemcpyAsync(&ovf, flags_.get() + 2, sizeof(int), hipMemcpyDeviceToHost, st_), "overflow");
-    check(hipStreamSynchronize(st_), "choose");
-    if (ovf) throw std::runtime_error("choose: chosen points exceed a segment's capacity");
+    if (nL < ns) {
+        check(hipMemcpyAsync(got, ci + status, sizeof(got), hipMemcpyDeviceToHost, st_), "choose status");
+        check(hipStreamSynchronize(st_), "choose");
+    }
+    if (got[0]) throw std::runtime_error("choose: chosen points exceed a segment's capacity");
     updateKeyBound();
     timers.chooseMs += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }

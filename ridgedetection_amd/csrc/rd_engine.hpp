@@ -303,8 +303,8 @@ private:
     DevBuf<int64_t> dN_, dM_;
     DevBuf<int> flags_;   // [0] allDone, [1] totalIters, [2] overflow
     // choose scratch
-    DevBuf<unsigned char> covered_;
-    std::vector<DevBuf<WorkItem>*> chooseItems_;
+    DevBuf<int> chooseInfo_;         // choose: large segments, their filter blocks and state
+    DevBuf<uint64_t> chooseOpen_;    // choose: samples of the large segments not decided yet
     // decimate scratch
     DevBuf<int> decInts_;
     DevBuf<int64_t> decI64_;

@@ -4,8 +4,8 @@
 //
 // The choose kernels (rd_choose.hip) need, beyond the points (input) and the chosen points,
 // indices and count (outputs), a few device words (the segment description, its radius, the
-// running count, an overflow flag), the work items of the chunked path and one "covered" byte
-// per sample.  Here they live in `scratch`, a fixed device array of this library, instead of
+// running count and cursor, an overflow flag) and one "open" bit per sample.  Here they live in
+// `scratch`, a fixed device array of this library, instead of
 // buffers a context allocates.  Every call on a device shares that device's copy of the array:
 // calls that overlap on one device (different streams, or threads) race and must be ordered by
 // the caller.  A call rewrites all of the array it reads before reading it, so nothing is
@@ -14,19 +14,15 @@
 #include "../../include/rdhip.h"
 #include "rd_choose.hpp"
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 
 namespace rdhip {
 namespace {
 
-constexpr int64_t kHeaderBytes = 256;                  // SegDesc, count, flags, radius
-constexpr int64_t kItemsBytes = 64 * sizeof(WorkItem); // one chunk's filter items (<= 64 x 1024 samples)
-constexpr int64_t kCoveredOff = 4096;                  // then one byte per sample
-constexpr int64_t kScratchBytes = kCoveredOff + RDHIP_NOALLOC_MAX_POINTS;
-
-static_assert(sizeof(SegDesc) + 16 + sizeof(double) <= kHeaderBytes, "header layout");
-static_assert(kHeaderBytes + kItemsBytes <= kCoveredOff, "items layout");
+constexpr int64_t kOpenOff = 4096;   // after the header, one bit per sample
+constexpr int64_t kScratchBytes = kOpenOff + RDHIP_NOALLOC_MAX_POINTS / 8;
 
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -34,13 +30,17 @@ struct Header {
     SegDesc seg;
     int segK;
     int overflow;
-    int segLarge;
-    int pad;
+    int largeSeg;       // 0: the one segment
+    int largeBlock[2];  // its filter blocks
+    int base;
+    int cursor;
+    int doneCount;
     double rSqr;   // read through segRSqr as the value type (float in the first 4 bytes)
 };
+static_assert(sizeof(Header) <= kOpenOff, "header layout");
 
 template <typename T>
-__global__ void noalloc_setup_kernel(unsigned char* base, int n, T rSqr, int large) {
+__global__ void noalloc_setup_kernel(unsigned char* base, int n, T rSqr) {
     if (threadIdx.x != 0) return;
     Header* h = reinterpret_cast<Header*>(base);
     SegDesc s{};
@@ -53,15 +53,13 @@ __global__ void noalloc_setup_kernel(unsigned char* base, int n, T rSqr, int lar
     h->seg = s;
     h->segK = 0;
     h->overflow = 0;
-    h->segLarge = large;
+    h->largeSeg = 0;
+    h->largeBlock[0] = 0;
+    h->largeBlock[1] = (n + kChooseBlock - 1) / kChooseBlock;
+    h->base = 0;
+    h->cursor = 0;
+    h->doneCount = 0;
     *reinterpret_cast<T*>(&h->rSqr) = rSqr;
-}
-
-// the filter items of chunk [c0, c1): 1024 samples each
-__global__ void noalloc_items_kernel(WorkItem* items, int c0, int c1) {
-    const int i = (int)threadIdx.x;
-    const int st = c0 + i * 1024;
-    if (st < c1) items[i] = WorkItem{0, st, min(c1, st + 1024), 0};
 }
 
 __global__ void noalloc_finish_kernel(const unsigned char* base, int32_t* count) {
@@ -96,24 +94,25 @@ hipError_t choose_noalloc(int dim, const T* points, int64_t n, int64_t stride, T
     hipError_t e = scratch_for_current_device(&base);
     if (e != hipSuccess) return e;
     Header* h = reinterpret_cast<Header*>(base);
-    WorkItem* items = reinterpret_cast<WorkItem*>(base + kHeaderBytes);
-    constexpr int kLarge = 32768;   // above this, the chunked path (as Engine::choose)
+    constexpr int kOneBlock = 4096;   // up to here one block takes the whole cloud (as Engine::choose)
     const int nn = (int)n;
-    const int large = nn > kLarge ? 1 : 0;
-    hipLaunchKernelGGL((noalloc_setup_kernel<T>), dim3(1), dim3(64), 0, st, base, nn, r * r, large);
+    hipLaunchKernelGGL((noalloc_setup_kernel<T>), dim3(1), dim3(64), 0, st, base, nn, r * r);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    ChooseArgs<T> a{points, stride, nullptr, chosen, chosenStride, &h->seg, 1, &h->segK,
-                    reinterpret_cast<const T*>(&h->rSqr), base + kCoveredOff, indices, &h->overflow, &h->segLarge};
-    if ((e = launch_choose_block<T>(a, dim, -1, 0, st)) != hipSuccess) return e;
-    if (large) {
-        if ((e = launch_choose_block<T>(a, dim, 0, 0, st)) != hipSuccess) return e;
-        for (int c = 1; choose_chunk_start(c) < nn; ++c) {
+    const ChooseArgs<T> a{points, stride, nullptr, chosen, chosenStride, &h->seg, 1, &h->segK,
+                          reinterpret_cast<const T*>(&h->rSqr), indices, &h->overflow, nullptr, 1, &h->largeSeg,
+                          h->largeBlock, reinterpret_cast<uint64_t*>(base + kOpenOff), &h->base, &h->cursor,
+                          &h->doneCount};
+    if (nn <= kOneBlock) {
+        if ((e = launch_choose_small<T>(a, dim, st)) != hipSuccess) return e;
+    } else {
+        // the number of rounds depends on the data and cannot be read back here: a fixed list of
+        // chunks instead, each filtered against every chosen point before it, then decided by one
+        // block however many batches that takes
+        for (int c = 0; choose_chunk_start(c) < nn; ++c) {
             const int c0 = choose_chunk_start(c), c1 = std::min(choose_chunk_start(c + 1), nn);
-            const int numItems = (c1 - c0 + 1023) / 1024;
-            hipLaunchKernelGGL(noalloc_items_kernel, dim3(1), dim3(64), 0, st, items, c0, c1);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-            if ((e = launch_choose_filter<T>(a, dim, items, numItems, st)) != hipSuccess) return e;
-            if ((e = launch_choose_block<T>(a, dim, c, 1, st)) != hipSuccess) return e;
+            const int blocks = (c1 - c0 + kChooseBlock - 1) / kChooseBlock;
+            if ((e = launch_choose_filter<T>(a, dim, c0 / kChooseBlock, blocks, true, st)) != hipSuccess) return e;
+            if ((e = launch_choose_resolve<T>(a, dim, c1, 0, st)) != hipSuccess) return e;
         }
     }
     hipLaunchKernelGGL(noalloc_finish_kernel, dim3(1), dim3(64), 0, st, base, count);
