@@ -151,25 +151,45 @@ __global__ __launch_bounds__(256) void dec_super_box_kernel(T* __restrict__ boxe
 
 // Row entries an element may keep from the count pass (provisional rows).
 constexpr int kDecProv = 32;
+// Waves that share the candidates of 64 elements.
+constexpr int kDecParts = 16;
+static_assert(kDecParts <= kDecProv, "a long row keeps its part counts in its provisional row");
 
 // Neighbour counts within r2 and 2 r2 of every element in its group (fill = 0), then the
-// CSR rows (fill = 1).  With prov, the count pass also writes each element's first kDecProv
-// row entries to prov[e][.]; rows that fit are copied into place (dec_prov_copy_kernel) and
-// the fill pass walks only the elements with longer rows.  A wave walks the union of its lanes' chunk ranges with wave-uniform
-// indices, so candidate coordinates and boxes are broadcast loads; each lane tests only the
-// candidates of its own group, in increasing element order, and only in chunks whose box
-// passes its own test, as a walk of its own would.
+// CSR rows (fill = 1).  A block takes 64 consecutive elements, one per lane; its waves (parts)
+// split the candidates, the union of the elements' group ranges, into consecutive runs.  With
+// prov, the count pass also collects each element's first kDecProv row entries in LDS, as the
+// waves find them, and writes them to prov[e][.] in increasing element order; rows that fit are
+// copied into place (dec_prov_copy_kernel).  A longer row keeps the parts' counts there instead,
+// from which the fill pass, which walks only such rows, starts each part.  A wave walks its run
+// with wave-uniform indices, so candidate coordinates and boxes are broadcast loads; each lane
+// tests only the candidates of its own group, in increasing element order, and only in chunks
+// whose box passes its own test, as a walk of its own would.
+//
+// Bound: VALU work, elements^2 pair tests where the order has no locality (boxes then exclude
+// nothing).  One wave per 64 elements left most of the chip idle: 300k 6-D points' ~15,000 chosen
+// points were 235 waves for 1024 SIMDs, 3.95 ms a pass; with 16 parts 0.31 ms.
 template <typename T, int DIM>
-__global__ __launch_bounds__(256) void dec_count_kernel(DecArgs a, const T* __restrict__ E,
-                                                        const T* __restrict__ groupRSqr, int fill,
-                                                        int64_t maxElems, const T* __restrict__ boxes,
-                                                        int64_t maxChunks, int* __restrict__ prov) {
+__global__ __launch_bounds__(kDecParts * kWave) void dec_count_kernel(DecArgs a, const T* __restrict__ E,
+                                                                     const T* __restrict__ groupRSqr, int fill,
+                                                                     int64_t maxElems, const T* __restrict__ boxes,
+                                                                     int64_t maxChunks, int* __restrict__ prov) {
+    __shared__ int part1[kDecParts][kWave], part2[kDecParts][kWave];
+    __shared__ int pool[kWave][kDecProv + 1];
+    __shared__ int poolCnt[kWave], selfHit[kWave];
     const int64_t total = *a.totalElems;
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= total && !fill && e <= maxElems) a.rowOff[e] = 0;   // tail of the offsets scan
+    const int lane = lane_id(), part = threadIdx.x / kWave;
+    const int parts = (int)blockDim.x / kWave;
+    const int64_t e = (int64_t)blockIdx.x * kWave + lane;
+    if (part == 0 && e >= total && !fill && e <= maxElems) a.rowOff[e] = 0;   // tail of the offsets scan
     // the fill pass skips the rows the provisional copy already wrote
-    const bool valid = e < total && !(fill && prov && a.c2[e] - 1 <= kDecProv);
-    if (__ballot(valid) == 0) return;   // no element of the wave needs a walk
+    const bool valid = e < total && !(fill && prov && a.rowOff[e + 1] - a.rowOff[e] <= kDecProv);
+    if (__ballot(valid) == 0) return;   // no element of the block needs a walk
+    const bool collect = !fill && prov != nullptr;
+    if (!fill) {
+        if (part == 0) poolCnt[lane] = selfHit[lane] = 0;
+        __syncthreads();
+    }
     int o = 0, n = 0;
     T rSqr = T(0), p[DIM];
 #pragma unroll
@@ -183,9 +203,13 @@ __global__ __launch_bounds__(256) void dec_count_kernel(DecArgs a, const T* __re
         for (int d = 0; d < DIM; ++d) p[d] = E[e * DIM + d];
     }
     const T r4 = T(4) * rSqr;
-    int c1 = 0, c2 = 0;
-    int w = fill && valid ? a.rowOff[e] : 0;
-    int np = 0;   // row entries found (count pass)
+    int c1 = 0;
+    int np = 0;   // row entries: neighbours within 2 r2 other than the element itself
+    int w = 0;
+    if (fill && valid) {
+        w = a.rowOff[e];
+        for (int q = 0; q < part; ++q) w += prov[e * kDecProv + q];
+    }
     // Chunks whose box lies farther than 2 r2 hold no neighbour: the squared distance to a
     // box bounds every member's from below; the margin covers the rounding of both sums.  A
     // super box holds its chunks' boxes, and every step of the box distance is monotone, so
@@ -210,6 +234,12 @@ __global__ __launch_bounds__(256) void dec_count_kernel(DecArgs a, const T* __re
     }
     wFirst = __builtin_amdgcn_readfirstlane(wFirst);
     wLast = __builtin_amdgcn_readfirstlane(wLast);
+    if (wFirst <= wLast) {   // this wave's run of chunks
+        const int64_t len = (int64_t)wLast - wFirst + 1;
+        const int f = __builtin_amdgcn_readfirstlane(wFirst + (int)(len * part / parts));
+        wLast = __builtin_amdgcn_readfirstlane(wFirst + (int)(len * (part + 1) / parts) - 1);
+        wFirst = f;
+    }
     for (int sc = wFirst / kDecSuper; wFirst <= wLast && sc <= wLast / kDecSuper; ++sc) {
         const bool wantS = any && sc >= cFirst / kDecSuper && sc <= cLast / kDecSuper &&
                            !(boxDist(boxes + (maxChunks + sc) * 2 * DIM) > skipAbove);
@@ -230,38 +260,59 @@ __global__ __launch_bounds__(256) void dec_count_kernel(DecArgs a, const T* __re
                     const bool in1 = dd <= rSqr;
                     const bool in2 = dd <= r4;
                     c1 += in1;
-                    c2 += in2;
-                    if (in2 && j != e) {
+                    if (in2 && j == e) {
+                        selfHit[lane] = 1;
+                    } else if (in2) {
                         const int v = (j << 1) | (in1 ? 1 : 0);
-                        if (fill)
-                            a.nbr[w++] = v;
-                        else if (prov && np < kDecProv)
-                            prov[e * kDecProv + np] = v;
                         ++np;
+                        if (fill) {
+                            a.nbr[w++] = v;
+                        } else if (collect) {
+                            const int at = atomicAdd(&poolCnt[lane], 1);
+                            if (at < kDecProv) pool[lane][at] = v;
+                        }
                     }
                 }
             }
         }
     }
-    if (!fill && valid) {
-        a.c1[e] = c1;
-        a.c2[e] = c2;
-        // neighbours other than itself (scanned to offsets); elements of a skipped group
-        // (n == 0) have no list at all
-        a.rowOff[e] = n > 0 ? c2 - 1 : 0;
+    if (fill) return;
+    part1[part][lane] = c1;
+    part2[part][lane] = np;
+    __syncthreads();
+    if (collect) {
+        // 16 threads an element: entry by entry to its rank (entries rise with the element index)
+        for (int x = (int)threadIdx.x; x < kWave * kDecProv; x += (int)blockDim.x) {
+            const int el = x / kDecProv, k = x % kDecProv;
+            const int cnt = poolCnt[el];
+            if (cnt > kDecProv || k >= cnt) continue;
+            const int v = pool[el][k];
+            int rank = 0;
+            for (int y = 0; y < cnt; ++y) rank += pool[el][y] < v;
+            prov[((int64_t)blockIdx.x * kWave + el) * kDecProv + rank] = v;
+        }
     }
+    if (part != 0 || !valid) return;
+    c1 = np = 0;
+    for (int q = 0; q < parts; ++q) {
+        c1 += part1[q][lane];
+        np += part2[q][lane];
+    }
+    a.c1[e] = c1;
+    a.c2[e] = np + selfHit[lane];
+    a.rowOff[e] = np;   // scanned to offsets (0 for the elements of a skipped group, whose n is 0)
+    if (collect && np > kDecProv)
+        for (int q = 0; q < parts; ++q) prov[e * kDecProv + q] = part2[q][lane];
 }
 
-// Copies the provisional rows that hold the whole row (c2 - 1 <= kDecProv) into the CSR.
+// Copies the provisional rows that hold the whole row (at most kDecProv entries) into the CSR.
 __global__ __launch_bounds__(256) void dec_prov_copy_kernel(DecArgs a, const int* __restrict__ prov) {
     const int64_t total = *a.totalElems;
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= total) return;
-    const int g = a.elemGroup[e];
-    if (a.groupCnt[g] <= 0) return;   // skipped group: no row
-    const int cnt = a.c2[e] - 1;
-    if (cnt > kDecProv) return;
     const int o = a.rowOff[e];
+    const int cnt = a.rowOff[e + 1] - o;
+    if (cnt > kDecProv) return;
     for (int k = 0; k < cnt; ++k) a.nbr[o + k] = prov[e * kDecProv + k];
 }
 
@@ -641,7 +692,8 @@ hipError_t decimate_groups(DecArgs& a, T* S, int64_t sStride, int dim, const T* 
     T* boxes = static_cast<T*>(ws.boxes);
     T* coords = boxes + (maxChunks + maxSupers) * 2 * dim;
     int* prov = useProv ? reinterpret_cast<int*>(static_cast<char*>(ws.boxes) + provOff) : nullptr;
-    const unsigned blocks = (unsigned)((maxElems + 1 + 255) / 256);
+    const unsigned blocks = (unsigned)((maxElems + kWave) / kWave);
+    const unsigned countThreads = (useProv ? kDecParts : 1) * kWave;
     bool ok = false;
     RD_DISPATCH_DIM(dim, {
         hipLaunchKernelGGL((dec_chunk_box_kernel<T, DIM>),
@@ -649,7 +701,7 @@ hipError_t decimate_groups(DecArgs& a, T* S, int64_t sStride, int dim, const T* 
                            (const T*)S, sStride, boxes, maxChunks, coords);
         hipLaunchKernelGGL((dec_super_box_kernel<T, DIM>), dim3((unsigned)((maxSupers + 255) / 256)), dim3(256), 0,
                            st, boxes, maxChunks, maxSupers);
-        hipLaunchKernelGGL((dec_count_kernel<T, DIM>), dim3(blocks), dim3(256), 0, st, a, (const T*)coords,
+        hipLaunchKernelGGL((dec_count_kernel<T, DIM>), dim3(blocks), dim3(countThreads), 0, st, a, (const T*)coords,
                            groupRSqr, 0, maxElems, (const T*)boxes, maxChunks, prov);
         ok = true;
     });
@@ -674,7 +726,7 @@ hipError_t decimate_groups(DecArgs& a, T* S, int64_t sStride, int dim, const T* 
         hipLaunchKernelGGL(dec_prov_copy_kernel, dim3((unsigned)((maxElems + 255) / 256)), dim3(256), 0, st, a,
                            (const int*)prov);
     RD_DISPATCH_DIM(dim, {
-        hipLaunchKernelGGL((dec_count_kernel<T, DIM>), dim3(blocks), dim3(256), 0, st, a, (const T*)coords,
+        hipLaunchKernelGGL((dec_count_kernel<T, DIM>), dim3(blocks), dim3(countThreads), 0, st, a, (const T*)coords,
                            groupRSqr, 1, maxElems, (const T*)boxes, maxChunks, prov);
     });
     // 4. ordered removal: small groups one wave each; large groups in dependency rounds
