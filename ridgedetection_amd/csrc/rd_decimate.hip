@@ -194,7 +194,8 @@ __global__ __launch_bounds__(kDecParts * kWave) void dec_count_kernel(DecArgs a,
     T rSqr = T(0), p[DIM];
 #pragma unroll
     for (int d = 0; d < DIM; ++d) p[d] = T(0);
-    if (valid) {
+    // ranges of all 64 elements, also of those the fill pass skips: both passes split the same runs
+    if (e < total) {
         const int g = a.elemGroup[e];
         o = a.groupOff[g];
         n = a.groupCnt[g];
@@ -224,8 +225,7 @@ __global__ __launch_bounds__(kDecParts * kWave) void dec_count_kernel(DecArgs a,
         }
         return bd;
     };
-    const bool any = valid && n > 0;
-    const int cFirst = any ? o / kDecChunk : INT_MAX, cLast = any ? (o + n - 1) / kDecChunk : -1;
+    const int cFirst = n > 0 ? o / kDecChunk : INT_MAX, cLast = n > 0 ? (o + n - 1) / kDecChunk : -1;
     int wFirst = cFirst, wLast = cLast;
 #pragma unroll
     for (int m = 1; m < kWave; m <<= 1) {
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(kDecParts * kWave) void dec_count_kernel(DecArgs a,
         wFirst = f;
     }
     for (int sc = wFirst / kDecSuper; wFirst <= wLast && sc <= wLast / kDecSuper; ++sc) {
-        const bool wantS = any && sc >= cFirst / kDecSuper && sc <= cLast / kDecSuper &&
+        const bool wantS = valid && n > 0 && sc >= cFirst / kDecSuper && sc <= cLast / kDecSuper &&
                            !(boxDist(boxes + (maxChunks + sc) * 2 * DIM) > skipAbove);
         if (__ballot(wantS) == 0) continue;
         const int cEnd = min(wLast, sc * kDecSuper + kDecSuper - 1);

@@ -32,3 +32,22 @@ def test_cluster_sizes(oracle, size, shuffled, rule, dtype):
     ref, kept = oracle.decimate(S, 0.1, nocopy=rule == 1)
     np.testing.assert_array_equal(np.flatnonzero(keep), kept)
     np.testing.assert_array_equal(SD, ref)
+
+
+@pytest.mark.parametrize("dim,dtype", [(2, np.float32), (3, np.float64)])
+def test_long_rows_of_many_groups(oracle, dim, dtype):
+    """Batches decimate per cloud: blocks of 64 elements hold several clouds' points, some with
+    rows longer than the provisional ones and some without."""
+    from ridgedetection_amd import synth
+    from ridgedetection_amd._lib import Context
+    g = np.random.Generator(np.random.PCG64(7 + dim))
+    clouds = []
+    for i in range(24):
+        P = synth.segment_chain(int(g.integers(300, 9000)), dim, seed=50 + i, sigma=0.03, dtype=dtype)
+        r1 = float(g.uniform(0.04, 0.12))
+        clouds.append((P, r1, float(g.uniform(2.0, 8.0)) * r1))
+    print(f"case decimate batch d={dim} {np.dtype(dtype).name}", flush=True)
+    with Context(dim, dtype) as c:
+        res = c.batch([p for p, _, _ in clouds], [a for _, a, _ in clouds], [b for _, _, b in clouds])
+    for (P, r1, r2), S in zip(clouds, res):
+        np.testing.assert_array_equal(S, oracle.ridge_detection(P, r1, r2)[0])
