@@ -31,21 +31,6 @@ namespace rdhip {
 
 namespace {
 
-__device__ __forceinline__ float read_lane(float v, int l) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-__device__ __forceinline__ double read_lane(double v, int l) {
-    const long long b = __double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(b & 0xffffffffLL), l);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), l);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-__device__ __forceinline__ uint64_t read_lane(uint64_t v, int l) {
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(v & 0xffffffffULL), l);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l);
-    return ((uint64_t)hi << 32) | lo;
-}
-
 // LDS of resolve_batch: the points the current wave chose, double buffered so that one barrier
 // separates a turn from the next.
 template <typename T, int DIM>

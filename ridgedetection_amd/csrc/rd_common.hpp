@@ -91,6 +91,22 @@ __device__ __forceinline__ int64_t point_of(const int* __restrict__ pIndex, int6
 __device__ __forceinline__ int lane_id() { return (int)__lane_id(); }
 __device__ __forceinline__ uint64_t lanes_below() { return __lanemask_lt(); }
 
+// lane l's value in every lane (l uniform), through an SGPR
+__device__ __forceinline__ float read_lane(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double read_lane(double v, int l) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(b & 0xffffffffLL), l);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ uint64_t read_lane(uint64_t v, int l) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(v & 0xffffffffULL), l);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l);
+    return ((uint64_t)hi << 32) | lo;
+}
+
 // XCD-aware block order: the GPU hands consecutive workgroups of a launch to its 8 XCDs in
 // turn, and each XCD has its own L2.  Block i of an n-block launch takes item xcd_item(i, n),
 // a bijection of [0, n) under which the blocks of one XCD take one contiguous run of items,

@@ -7,6 +7,7 @@
 // segments in one launch per kernel; all counts stay on the device and the host reads
 // them back once per round (or once every few evolve iterations to test convergence).
 #include "rd_engine.hpp"
+#include "rd_serialsum.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -413,7 +414,7 @@ void Engine<T>::ensureEvolveScratch() {
     moved_.reserve((size_t)slots * dim_);
     sums_.reserve((size_t)sStride_ * dim_);
     sortWs_.reserve(sort_workspace_bytes(totalP, (int)std::max<int64_t>(totalSlots_, 2)));
-    sortedP_.reserve((size_t)totalP * dim_);
+    sortedP_.reserve((size_t)totalP * dim_ + kSerialSlack);
     xTable_.reserve((size_t)(dim_ + 1) * std::max<int64_t>(sStride_, 1));
     segX_.reserve((size_t)std::max<size_t>(segs_.size(), 1) * kScreenStride);
     check(hipMemcpyAsync(dN_.get(), &totalP, sizeof(int64_t), hipMemcpyHostToDevice, st_), "n");
@@ -460,7 +461,7 @@ void Engine<T>::ensureChainScratch() {
     chainTotalPos_.reserve(1);
     chainHist_.reserve((size_t)std::max<int64_t>(h, 1));
     chainTotals_.reserve((size_t)rows);
-    if (sortedP_.n < (size_t)(m * dim_)) sortedP_.reserve((size_t)(m * dim_));
+    if (sortedP_.n < (size_t)(m * dim_) + kSerialSlack) sortedP_.reserve((size_t)(m * dim_) + kSerialSlack);
     const int64_t entries = kLongWaves;   // the length-based wave list (at most kLongWaves / dim used)
     if (longList_.n < (size_t)entries) longList_.reserve((size_t)entries);
     chainLongIdx_.reserve((size_t)std::max<int64_t>(totalSlots_, 1));

@@ -20,12 +20,12 @@
 //      bit-identical), applies the shift rule and raises the segment's "moved" flag.
 //      Chains holding a sorted position that is a multiple of L (every chain of at least L
 //      members; L adapts so that at most kLongWaves entries are needed), or listed by length,
-//      go to a block of four waves each instead, in the same launch: each wave sums a quarter
-//      of the chain from 64 speculative starts at once, one per lane, and the quarter whose
-//      start matches the exact sum before it is kept (chain_sum_parts).
+//      go to a wave each instead, in the same launch, which computes the same serial sum in
+//      parallel (rd_serialsum.hpp).
 //   5. evolve_finalize -- per-segment iteration count and convergence; global all-done.
 #include "rd_evolve.hpp"
 #include "rd_rowsum.hpp"
+#include "rd_serialsum.hpp"
 
 namespace rdhip {
 
@@ -81,18 +81,16 @@ __global__ __launch_bounds__(256) void gather_members_kernel(const T* __restrict
 // depends only on that coordinate's sum (rd/cpu/brute_force/evolve.hpp:129-179).
 // ---------------------------------------------------------------------------------
 // ---------------------------------------------------------------------------------
-// 4b'. ordered sums through LDS: a group of kLanes lanes (a whole wave, or a 16-lane row)
-// sums one chain.  Tiles of kLanes * kLongPer members are loaded coalesced one tile before
-// their turn (the loads of tile t + 1 are in flight while tile t is summed), staged in the
-// group's LDS slice and added in member order by every lane of the group from broadcast
-// LDS reads, so each member costs one plain dependent add (6.25 cycles, against 13.25 for
-// an add fed by a DPP row broadcast).  Members past the end of the chain are staged as +0
+// 4b'. ordered sums through LDS: a 16-lane row sums one chain.  Tiles of 256 members are loaded
+// coalesced one tile before their turn (the loads of tile t + 1 are in flight while tile t is
+// summed), staged in the row's LDS slice and added in member order by every lane of the row from
+// broadcast LDS reads, so each member costs one plain dependent add (6.25 cycles, against 13.25
+// for an add fed by a DPP row broadcast).  Members past the end of the chain are staged as +0
 // (see above).  The four rows of a wave read four slices whose starts differ by 16 bytes
 // modulo the bank width, so their broadcasts do not collide.
 // ---------------------------------------------------------------------------------
-constexpr int kLongPer = 16;
-constexpr int kLongTile = kLongPer * kWave;
-constexpr int kRowTile = kLongPer * 16;
+constexpr int kRowPer = 16;
+constexpr int kRowTile = kRowPer * 16;
 
 template <typename T>
 struct WideOf;
@@ -101,10 +99,10 @@ struct WideOf<float> { using type = float4; static constexpr int n = 4; };
 template <>
 struct WideOf<double> { using type = double2; static constexpr int n = 2; };
 
-// LDS per wave: one wave slice, or four row slices padded by one wide read each
+// LDS per wave: four row slices padded by one wide read each
 template <typename T>
 constexpr int wave_lds_elems() {
-    return kLongTile > 4 * (kRowTile + WideOf<T>::n) ? kLongTile : 4 * (kRowTile + WideOf<T>::n);
+    return 4 * (kRowTile + WideOf<T>::n);
 }
 
 // sum + v.x + v.y (+ v.z + v.w), in that order
@@ -126,78 +124,58 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Serial sum start + src[0] + src[1] + ... + src[cnt - 1] by a group of kLanes lanes (every
-// lane of the wave takes part; `steps` is the wave-uniform largest cnt of its groups); tile is
-// the group's LDS slice.  `start` may differ between lanes (each lane then returns its own sum)
-// and must not be -0 (the zeros of the first pass and of the padding leave any other value as
-// it is).  load(0) may be issued early (the first tile's members are then in reg) and the sum
-// run later.
-template <typename T, int kLanes>
-struct OrderedRun {
-    static constexpr int kTile = kLanes * kLongPer;
-    const T* __restrict__ src;
-    int cnt, last, lane;
-    T reg[kLongPer];
-
-    __device__ __forceinline__ OrderedRun(const T* __restrict__ s, int n)
-        : src(s), cnt(n), last(max(n - 1, 0)), lane((int)(threadIdx.x & (kLanes - 1))) {}
-
+// Serial sum src[0] + src[1] + ... + src[cnt - 1] by a row of 16 lanes (every lane of the wave
+// takes part; `steps` is the wave-uniform largest cnt of its rows); tile is the row's LDS slice.
+template <typename T>
+__device__ __forceinline__ T row_lds_sum(const T* __restrict__ src, int cnt, int steps, T* tile) {
+    const int last = max(cnt - 1, 0), lane = (int)(threadIdx.x & 15);
+    T reg[kRowPer];
     // tile t: index clamped into the chain and masked (tile t + 1 is loaded after tile t is
     // staged; its loads are not waited for before tile t's sum)
-    __device__ __forceinline__ void load(int t) {
+    auto load = [&](int t) {
 #pragma unroll
-        for (int c = 0; c < kLongPer; ++c) {
-            const int i = t * kTile + c * kLanes + lane;
+        for (int c = 0; c < kRowPer; ++c) {
+            const int i = t * kRowTile + c * 16 + lane;
             const T x = src[min(i, last)];
             reg[c] = i < cnt ? x : T(0);
         }
-    }
-
-    // the sum, with tile 0 already in reg
-    __device__ __forceinline__ T run(int steps, T* tile, T start) {
-        using W = typename WideOf<T>::type;
-        constexpr int kW = WideOf<T>::n;
-        const int nTiles = (steps + kTile - 1) / kTile;
-        T sum = start;
-        for (int t = 0; t < nTiles; ++t) {
-            wave_lds_sync();
+    };
+    load(0);
+    using W = typename WideOf<T>::type;
+    constexpr int kW = WideOf<T>::n;
+    const int nTiles = (steps + kRowTile - 1) / kRowTile;
+    T sum = T(0);
+    for (int t = 0; t < nTiles; ++t) {
+        wave_lds_sync();
 #pragma unroll
-            for (int c = 0; c < kLongPer; ++c) tile[c * kLanes + lane] = reg[c];
-            wave_lds_sync();
-            load(t + 1);
-            // groups of kG wide reads: group g + 1 is read while group g is added (the first
-            // pass adds a group of zeros, which leaves the sum unchanged); the scheduling
-            // barriers keep the reads a whole group ahead of their adds
-            const W* w = reinterpret_cast<const W*>(tile);
-            constexpr int kG = 8, kNQ = kTile / kW;
-            static_assert(kNQ % kG == 0, "tile is not a whole number of read groups");
-            W cur[kG];
+        for (int c = 0; c < kRowPer; ++c) tile[c * 16 + lane] = reg[c];
+        wave_lds_sync();
+        load(t + 1);
+        // groups of kG wide reads: group g + 1 is read while group g is added (the first
+        // pass adds a group of zeros, which leaves the sum unchanged); the scheduling
+        // barriers keep the reads a whole group ahead of their adds
+        const W* w = reinterpret_cast<const W*>(tile);
+        constexpr int kG = 8, kNQ = kRowTile / kW;
+        static_assert(kNQ % kG == 0, "tile is not a whole number of read groups");
+        W cur[kG];
 #pragma unroll
-            for (int g = 0; g < kG; ++g) cur[g] = W{};
+        for (int g = 0; g < kG; ++g) cur[g] = W{};
 #pragma unroll 2
-            for (int q0 = 0; q0 < kNQ; q0 += kG) {
-                W nxt[kG];
+        for (int q0 = 0; q0 < kNQ; q0 += kG) {
+            W nxt[kG];
 #pragma unroll
-                for (int g = 0; g < kG; ++g) nxt[g] = w[q0 + g];
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int g = 0; g < kG; ++g) sum = add_wide(sum, cur[g]);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int g = 0; g < kG; ++g) cur[g] = nxt[g];
-            }
+            for (int g = 0; g < kG; ++g) nxt[g] = w[q0 + g];
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int g = 0; g < kG; ++g) sum = add_wide(sum, cur[g]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < kG; ++g) cur[g] = nxt[g];
         }
-        return sum;
+#pragma unroll
+        for (int g = 0; g < kG; ++g) sum = add_wide(sum, cur[g]);
     }
-};
-
-template <typename T, int kLanes>
-__device__ __forceinline__ T group_ordered_sum(const T* __restrict__ src, int cnt, int steps, T* tile, T start) {
-    OrderedRun<T, kLanes> r(src, cnt);
-    r.load(0);
-    return r.run(steps, tile, start);
+    return sum;
 }
 
 // ---------------------------------------------------------------------------------
@@ -337,157 +315,115 @@ __device__ __forceinline__ void chain_sum_rows(const ShiftArgs<T>& a, int64_t bl
     }
     const int steps = wave_row_max(cnt);
     const int rowInWave = (threadIdx.x & (kWave - 1)) / kRow;
-    const T sum = group_ordered_sum<T, kRow>(src, cnt, steps, waveLds + rowInWave * (kRowTile + WideOf<T>::n), T(0));
+    const T sum = row_lds_sum(src, cnt, steps, waveLds + rowInWave * (kRowTile + WideOf<T>::n));
     if (seg < 0 || t != 0) return;
     shift_coordinate(a, d, slot, seg, cnt, sum);
 }
 
-// Ordered integer of a value (the order of the values, -0 and +0 both 0) and back (never -0).
-__device__ __forceinline__ int64_t ord_of(float x) {
-    const int i = __float_as_int(x);
-    return i >= 0 ? (int64_t)i : -(int64_t)(i & 0x7fffffff);
-}
-__device__ __forceinline__ int64_t ord_of(double x) {
-    const long long i = __double_as_longlong(x);
-    return i >= 0 ? (int64_t)i : -(int64_t)(i & 0x7fffffffffffffffLL);
-}
+// A listed chain: its slot, segment and member range; false when the entry is not live.
+struct ListedChain {
+    int slot, seg, off, cnt;
+};
 template <typename T>
-__device__ __forceinline__ T from_ord(int64_t o);
-template <>
-__device__ __forceinline__ float from_ord<float>(int64_t o) {
-    return __int_as_float(o >= 0 ? (int)o : (int)(0x80000000u | (unsigned)(-o)));
-}
-template <>
-__device__ __forceinline__ double from_ord<double>(int64_t o) {
-    return __longlong_as_double(o >= 0 ? (long long)o : (long long)(0x8000000000000000ULL | (unsigned long long)(-o)));
-}
-__device__ __forceinline__ bool same_bits(float a, float b) { return __float_as_uint(a) == __float_as_uint(b); }
-__device__ __forceinline__ bool same_bits(double a, double b) {
-    return __double_as_longlong(a) == __double_as_longlong(b);
+__device__ __forceinline__ bool listed_chain(const ShiftArgs<T>& a, int64_t e, ListedChain& c) {
+    // the list entry is loaded with the live count (in bounds either way: e < the list's
+    // capacity), and the chain's range and segment together once the entry is known to be live
+    const int key = a.longList[e];
+    if (a.longCount ? e >= min(*a.longCount, a.longCap) : (e << a.longShift) >= *a.mPtr) return false;
+    if (key < 0) return false;
+    c.slot = a.denseChains ? a.rowSlots[key] : key;
+    c.seg = a.slotSeg[c.slot];
+    c.off = a.chainOff[key];
+    c.cnt = a.chainEnd[key] - c.off;
+    // a chain listed by length belongs to a live segment and a live slot (the member scatter
+    // lists no other); a chain listed by position is checked
+    return a.longCount || !(c.seg < 0 || a.segDone[c.seg] || (int)(c.slot - a.segs[c.seg].sOff) >= a.segK[c.seg]);
 }
 
-// Long chains: one block of kParts waves per (list entry, coordinate).  The serial sum of a
-// chain is cut into kParts runs of consecutive members, one per wave, summed at the same time:
-// wave p cannot know the exact partial sum its run starts from (the serial sum of every member
-// before it), so each of its 64 lanes sums the run from its own start, the 64 consecutive values
-// of the type centred on the correctly rounded sum of those members (from the wider sums of the
-// runs before it).  Wave 0 then walks the runs in order: run p's result is the one of the lane
-// whose start equals, bit for bit, the exact sum through run p - 1 -- the same adds of the same
-// values in the same order as one serial sum, so the same result.  When no lane started from that
-// value (the rounding errors of the serial sum before run p exceed 32 units of its last place,
-// about one run in five hundred), wave 0 sums run p again from it.  The result never depends on
-// the estimate; only the time does.
-constexpr int kParts = 256 / kWave;
+// Long chains, exact: one wave per (list entry, coordinate), four to a block (rd_serialsum.hpp); the
+// sums that hover around zero are finished one after the other by the whole block.
+constexpr int kHoverMin = 1024;   // values left that pay for the block's turn
 
 template <typename T>
-struct PartLds {
-    typename WideSum<T>::Acc wide[kParts];
-    int64_t ordE[kParts];
-    T cand[kParts][kWave];
-    T start[kParts][kWave];
+struct HoverLds {
+    int n;
+    int64_t entry[256 / kWave];
+    PartialSum<T> part[256 / kWave];
+    RunLds<T, WideSum<T>> runs;
 };
 
 template <typename T, int DIM>
-__device__ __forceinline__ void chain_sum_parts(const ShiftArgs<T>& a, int64_t entry, T* tile, PartLds<T>& sh) {
-    using W = WideSum<T>;
-    using Run = OrderedRun<T, kWave>;
-    const int64_t e = entry / DIM;
-    const int d = (int)(entry - e * DIM);
-    // every exit before the barriers below is the same for the whole block.  The list entry is
-    // loaded with the live count (in bounds either way: e < the list's capacity), and the chain's
-    // range and segment together once the entry is known to be live.
-    const int key = a.longList[e];
-    if (a.longCount ? e >= min(*a.longCount, a.longCap) : (e << a.longShift) >= *a.mPtr) return;
-    if (key < 0) return;
-    const int slot = a.denseChains ? a.rowSlots[key] : key;
-    const int seg = a.slotSeg[slot];
-    const int off = a.chainOff[key];
-    const int cnt = a.chainEnd[key] - off;
-    // a chain listed by length belongs to a live segment and a live slot (the member scatter
-    // lists no other); a chain listed by position is checked
-    if (!a.longCount && (seg < 0 || a.segDone[seg] || (int)(slot - a.segs[seg].sOff) >= a.segK[seg])) return;
-    const T* __restrict__ base = a.sortedP + (int64_t)d * a.mStride + off;
-    const int w = threadIdx.x / kWave, lane = lane_id();
-    if (a.tolerance) {
-        // a quarter of the chain per wave in the wider type, combined in a fixed order
-        const int q0 = (int)((int64_t)cnt * w / kParts), q1 = (int)((int64_t)cnt * (w + 1) / kParts);
-        const typename W::Acc part = group_parallel_sum<T, kWave>(base + (q1 > q0 ? q0 : 0), q1 - q0);
-        if (lane == 0) sh.wide[w] = part;
-        __syncthreads();
-        if (w != 0) return;
-        typename W::Acc total = W::zero();
-        for (int q = 0; q < kParts; ++q) total = W::add(total, sh.wide[q]);
-        if (lane == 0) shift_coordinate_wide(a, d, slot, seg, cnt, W::value(total));
-        return;
-    }
-    auto run_of = [&](int p, int& n) {
-        const int b0 = (int)((int64_t)cnt * p / kParts);
-        n = (int)((int64_t)cnt * (p + 1) / kParts) - b0;
-        return base + (n > 0 ? b0 : 0);   // an empty run reads (and discards) the chain's first member
-    };
-    int n;
-    const T* __restrict__ src = run_of(w, n);
-    // the run's first tile, then the wider sum of the whole run from those registers and the
-    // loads of the rest, issued before any of them is waited for
-    Run run(src, n);
-    run.load(0);
-    typename W::Acc acc[4] = {W::zero(), W::zero(), W::zero(), W::zero()};
-    for (int i0 = Run::kTile; i0 < n; i0 += Run::kTile) {
-        T v[kLongPer];
-#pragma unroll
-        for (int c = 0; c < kLongPer; ++c) {
-            const int i = i0 + c * kWave + lane;
-            v[c] = i < n ? src[i] : T(0);
-        }
-#pragma unroll
-        for (int c = 0; c < kLongPer; ++c) acc[c & 3] = W::add(acc[c & 3], v[c]);
-    }
-#pragma unroll
-    for (int c = 0; c < kLongPer; ++c) acc[c & 3] = W::add(acc[c & 3], run.reg[c]);
-    typename W::Acc wide = W::add(W::add(acc[0], acc[1]), W::add(acc[2], acc[3]));
-#pragma unroll
-    for (int m = kWave / 2; m >= 1; m /= 2) wide = W::add(wide, W::xorShfl(wide, m));
-    if (lane == 0) sh.wide[w] = wide;
+__device__ __forceinline__ void chain_sum_waves(const ShiftArgs<T>& a, int64_t entry, int64_t entries,
+                                                HoverLds<T>& sh) {
+    if (threadIdx.x == 0) sh.n = 0;
     __syncthreads();
-    T start = T(0);
-    if (w > 0) {
-        typename W::Acc est = W::zero();
-        for (int q = 0; q < w; ++q) est = W::add(est, sh.wide[q]);
-        const T e0 = (T)W::value(est);
-        const int64_t oe = ord_of(e0);
-        start = isfinite(e0) ? from_ord<T>(oe + lane - kWave / 2) : T(0);
-        if (lane == 0) sh.ordE[w] = oe;
-    }
-    const T cand = run.run(n, tile, start);
-    sh.cand[w][lane] = cand;
-    sh.start[w][lane] = start;
-    __syncthreads();
-    if (w != 0) return;
-    T x = sh.cand[0][0];
-    for (int p = 1; p < kParts; ++p) {
-        const int64_t o = ord_of(x) - sh.ordE[p] + kWave / 2;
-        if (o >= 0 && o < kWave && same_bits(sh.start[p][o], x)) {
-            x = sh.cand[p][o];
-        } else {
-            int np;
-            const T* __restrict__ sp = run_of(p, np);
-            x = group_ordered_sum<T, kWave>(sp, np, np, tile, x);
+    ListedChain c;
+    if (entry < entries && listed_chain(a, entry / DIM, c)) {
+        const int d = (int)(entry % DIM);
+        const PartialSum<T> p =
+            wave_serial_sum<T>(a.sortedP + (int64_t)d * a.mStride + c.off, c.cnt, kHoverMin);
+        if (lane_id() == 0) {
+            if (p.done >= c.cnt) {
+                shift_coordinate(a, d, c.slot, c.seg, c.cnt, p.sum);
+            } else {
+                const int at = atomicAdd(&sh.n, 1);
+                sh.entry[at] = entry;
+                sh.part[at] = p;
+            }
         }
     }
-    if (lane == 0) shift_coordinate(a, d, slot, seg, cnt, x);
+    __syncthreads();
+    for (int k = 0; k < sh.n; ++k) {
+        const int64_t en = sh.entry[k];
+        const PartialSum<T> p = sh.part[k];
+        const int d = (int)(en % DIM);
+        (void)listed_chain(a, en / DIM, c);
+        const T sum = block_speculative_sum<T, WideSum<T>>(a.sortedP + (int64_t)d * a.mStride + c.off + p.done,
+                                                           c.cnt - p.done, p.sum, sh.runs);
+        if (threadIdx.x == 0) shift_coordinate(a, d, c.slot, c.seg, c.cnt, sum);
+    }
 }
 
-// blocks [0, rowBlocks): 16-lane rows; the rest: one listed chain and coordinate each.  The
-// convergence bookkeeping follows in a launch of its own (evolve_finalize_kernel).
+// Long chains in tolerance mode: one block per (list entry, coordinate), a quarter of the chain
+// per wave in the wider type, the quarters added in order.
+constexpr int kParts = 256 / kWave;
+
 template <typename T, int DIM>
-__global__ __launch_bounds__(256) void chain_sum_shift_kernel(ShiftArgs<T> a, int64_t rowBlocks) {
+__device__ __forceinline__ void chain_sum_quarters(const ShiftArgs<T>& a, int64_t entry,
+                                                   typename WideSum<T>::Acc* quarter) {
+    using W = WideSum<T>;
+    const int64_t e = entry / DIM;
+    const int d = (int)(entry - e * DIM);
+    ListedChain c;
+    if (!listed_chain(a, e, c)) return;   // the same for the whole block
+    const T* __restrict__ base = a.sortedP + (int64_t)d * a.mStride + c.off;
+    const int w = threadIdx.x / kWave, lane = lane_id();
+    const int q0 = (int)((int64_t)c.cnt * w / kParts), q1 = (int)((int64_t)c.cnt * (w + 1) / kParts);
+    const typename W::Acc part = group_parallel_sum<T, kWave>(base + (q1 > q0 ? q0 : 0), q1 - q0);
+    if (lane == 0) quarter[w] = part;
+    __syncthreads();
+    if (w != 0) return;
+    typename W::Acc total = W::zero();
+    for (int q = 0; q < kParts; ++q) total = W::add(total, quarter[q]);
+    if (lane == 0) shift_coordinate_wide(a, d, c.slot, c.seg, c.cnt, W::value(total));
+}
+
+// blocks [0, rowBlocks): 16-lane rows; the rest: four listed (chain, coordinate) pairs each, one
+// per wave (tolerance mode: one pair).  The convergence bookkeeping follows in a launch of its own
+// (evolve_finalize_kernel).
+template <typename T, int DIM>
+__global__ __launch_bounds__(256) void chain_sum_shift_kernel(ShiftArgs<T> a, int64_t rowBlocks, int64_t entries) {
     __shared__ __align__(16) T tiles[256 / kWave][wave_lds_elems<T>()];
-    __shared__ PartLds<T> parts;
+    __shared__ typename WideSum<T>::Acc quarter[kParts];
+    __shared__ HoverLds<T> hover;
     if (*a.allDone) return;
-    if ((int64_t)blockIdx.x < rowBlocks)
+    if ((int64_t)blockIdx.x < rowBlocks) {
         chain_sum_rows<T, DIM>(a, blockIdx.x, tiles[threadIdx.x / kWave]);
-    else
-        chain_sum_parts<T, DIM>(a, (int64_t)blockIdx.x - rowBlocks, tiles[threadIdx.x / kWave], parts);
+    } else if (a.tolerance) {
+        chain_sum_quarters<T, DIM>(a, (int64_t)blockIdx.x - rowBlocks, quarter);
+    } else {
+        chain_sum_waves<T, DIM>(a, ((int64_t)blockIdx.x - rowBlocks) * kParts + threadIdx.x / kWave, entries, hover);
+    }
 }
 
 // ---------------------------------------------------------------------------------
@@ -523,9 +459,9 @@ template <typename T>
 hipError_t launch_chain_sum_shift(const ShiftArgs<T>& a, int dim, int64_t maxM, bool gather, hipStream_t st) {
     const int64_t rowBlocks = ((int64_t)dim * a.totalSlots + 15) / 16;
     if (rowBlocks <= 0) return hipSuccess;
-    const int64_t waves = a.longCount ? (int64_t)dim * a.longCap
-                                      : a.longList ? (int64_t)dim * long_list_entries(maxM, a.longShift) : 0;
-    const int64_t blocks = rowBlocks + waves;
+    const int64_t entries = a.longCount ? (int64_t)dim * a.longCap
+                                        : a.longList ? (int64_t)dim * long_list_entries(maxM, a.longShift) : 0;
+    const int64_t blocks = rowBlocks + (a.tolerance ? entries : (entries + kParts - 1) / kParts);
     const unsigned gblocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>((maxM + 255) / 256, 8192));
     bool ok = false;
     RD_DISPATCH_DIM(dim, {
@@ -533,7 +469,7 @@ hipError_t launch_chain_sum_shift(const ShiftArgs<T>& a, int dim, int64_t maxM, 
             hipLaunchKernelGGL((gather_members_kernel<T, DIM>), dim3(gblocks), dim3(256), 0, st, a.P, a.pStride,
                                a.pIndex, a.members, a.mPtr, a.sortedP, a.mStride, a.allDone);
         hipLaunchKernelGGL((chain_sum_shift_kernel<T, DIM>), dim3((unsigned)blocks), dim3(256), 0, st, a,
-                           rowBlocks);
+                           rowBlocks, entries);
         ok = true;
     });
     return ok ? hipGetLastError() : hipErrorInvalidValue;
