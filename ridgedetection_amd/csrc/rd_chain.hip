@@ -73,7 +73,21 @@ __global__ __launch_bounds__(256) void key_prefix_kernel(ChainArgs<T> a) {
     const int k = row - a.segRowOff[s];
     const SegDesc sd = a.segs[s];
     const int nb = (sd.nP + a.itemSize - 1) / a.itemSize;
-    int* __restrict__ r = a.hist + a.segHistOff[s] + (int64_t)k * nb;
+    if (a.act) {
+        // incremental: a chain whose members are the last iteration's keeps its total and is left
+        // out of this iteration's ordering and sums
+        const int64_t slot = sd.sOff + k;
+        const bool live = !a.segDone[s] && k < min(a.segK[s], a.segKeyCap[s]);
+        const int t = live && (a.allTouched || a.touched[slot]) ? 1 : 0;
+        if (lane == 0 && live) {
+            a.act[slot] = t;
+            a.touched[slot] = 0;
+            a.moved[slot] = 0;
+        }
+        if (live && !t) return;
+    }
+    const int* r = a.hist + a.segHistOff[s] + (int64_t)k * nb;
+    int* w = a.prefix + a.segHistOff[s] + (int64_t)k * nb;
     constexpr int kPer = 16;   // one pass for up to 1024 blocks
     int carry = 0;
     for (int base = 0; base < nb; base += kWave * kPer) {
@@ -100,7 +114,7 @@ __global__ __launch_bounds__(256) void key_prefix_kernel(ChainArgs<T> a) {
         int run = carry + incl - sum;
 #pragma unroll
         for (int j = 0; j < kPer; ++j) {
-            if (i0 + j < nb) r[i0 + j] = run;
+            if (i0 + j < nb) w[i0 + j] = run;
             run += v[j];
         }
         carry += __shfl(incl, kWave - 1);
@@ -153,13 +167,27 @@ __global__ __launch_bounds__(W * kWave) void member_scatter_kernel(ChainArgs<T> 
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         const int i = it.start + (wave * C + c) * kWave + lane;
-        const bool in = i < it.end;
-        lraw[c] = in ? lab[i] : -1;
-        const int64_t n = point_of(a.pIndex, sd.pOff + (in ? i : it.start));
+        lraw[c] = i < it.end ? lab[i] : -1;
+    }
+    if (a.act) {
+        // incremental: members of the chains ordered this iteration only
+        bool any = false;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            if (lraw[c] >= 0 && !a.act[lraw[c]]) lraw[c] = -1;
+            any = any || lraw[c] >= 0;
+        }
+        // the segment's first block also writes the chain ranges
+        if (!__syncthreads_or(any) && col != 0) return;
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int i = it.start + (wave * C + c) * kWave + lane;
+        const int64_t n = point_of(a.pIndex, sd.pOff + (i < it.end ? i : it.start));
 #pragma unroll
         for (int d = 0; d < DIM; ++d) p[c][d] = a.P[d * a.pStride + n];
     }
-    const int* __restrict__ hcol = a.hist + a.segHistOff[s] + col;
+    const int* __restrict__ hcol = a.prefix + a.segHistOff[s] + col;
     int tk[kMaxKeysPerThread], hv[kMaxKeysPerThread];
 #pragma unroll
     for (int j = 0; j < kMaxKeysPerThread; ++j) {
@@ -192,6 +220,7 @@ __global__ __launch_bounds__(W * kWave) void member_scatter_kernel(ChainArgs<T> 
                     const int64_t slot = sd.sOff + k;
                     a.chainOff[slot] = (int)base;
                     a.chainEnd[slot] = (int)(memberOff + end);
+                    if (a.act && !a.act[slot]) continue;
                     // long chains take a place in the wave list (which place does not matter:
                     // a chain's sum is the same on either path)
                     if (tk[j] >= a.longMin) {

@@ -60,6 +60,14 @@ struct ChainArgs {
     int* longIdx;
     int longMin;
     int longCap;
+    int* prefix;                // the exclusive prefixes: hist itself, or (incremental) a table like it
+    // incremental iterations (rd_spatial.hip), per slot: touched -- the chains to order (taken and
+    // cleared by the prefix pass; all of them when allTouched), act -- the chains ordered this
+    // iteration, moved -- cleared for the sums; null otherwise
+    int* touched;
+    int* act;
+    int* moved;
+    int allTouched;
 };
 
 // Launches the per-key prefix and the member scatter after a histogram scan over numItems

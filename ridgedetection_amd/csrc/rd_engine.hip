@@ -23,6 +23,8 @@ namespace {
 constexpr int kChooseFewSegs = 256;        // one block per CU
 constexpr int kChooseLargeFew = 4096;
 constexpr int kChooseLargeMany = 32768;
+constexpr double kIncMinKeys = 48;   // chosen points per segment (mean over samples)
+constexpr int kIncMinIters = 4;
 
 inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
@@ -136,7 +138,7 @@ template <typename T>
 T* Engine<T>::reservePoints(int64_t n) {
     if (n < 0) throw std::invalid_argument("negative point count");
     ++version_;
-    psegValid_ = false;
+    psegValid_ = spatialValid_ = false;
     nPoints_ = n;
     pStride_ = round_up(std::max<int64_t>(n, 1), 64);
     P_.reserve((size_t)pStride_ * dim_);
@@ -147,7 +149,7 @@ template <typename T>
 void Engine<T>::setPoints(const T* src, int64_t n, int layout, int64_t stride, bool onDevice) {
     if (n < 0) throw std::invalid_argument("negative point count");
     ++version_;
-    psegValid_ = false;
+    psegValid_ = spatialValid_ = false;
     nPoints_ = n;
     pStride_ = round_up(std::max<int64_t>(n, 1), 64);
     P_.reserve((size_t)pStride_ * dim_);
@@ -191,6 +193,11 @@ template <typename T>
 void Engine<T>::setSegments(const std::vector<SegDesc>& segs, const std::vector<int64_t>& capacities,
                             const std::vector<T>& r1, const std::vector<T>& r2, bool indexed) {
     const int ns = (int)segs.size();
+    // the spatial order of unindexed samples depends on the points and the segments' ranges only
+    bool sameRanges = !indexed && !useIndex_ && segs.size() == segs_.size();
+    for (int s = 0; s < ns && sameRanges; ++s)
+        sameRanges = segs[s].pOff == segs_[s].pOff && segs[s].nP == segs_[s].nP;
+    spatialValid_ = spatialValid_ && sameRanges;
     useIndex_ = indexed;
     psegValid_ = false;
     if (capacities.size() != segs.size() || r1.size() != segs.size() || r2.size() != segs.size())
@@ -308,6 +315,17 @@ void Engine<T>::rebuildActive(const std::vector<int>& segDone) {
         check(hipMemcpyAsync(dItems_.get(), act.data(), sizeof(WorkItem) * n, hipMemcpyHostToDevice, st_), "items");
     check(hipMemcpyAsync(flags_.get() + 4, &n, sizeof(int), hipMemcpyHostToDevice, st_), "items");
     check(hipMemcpyAsync(dN_.get(), &off, sizeof(int64_t), hipMemcpyHostToDevice, st_), "n");
+    std::vector<WorkItem> box;
+    int nBox = 0;
+    if (incNow_) {
+        for (const WorkItem& it : boxItems_)
+            if (!segDone[it.seg]) box.push_back(it);
+        nBox = (int)box.size();
+        if (nBox > 0)
+            check(hipMemcpyAsync(dBoxItems_.get(), box.data(), sizeof(WorkItem) * nBox, hipMemcpyHostToDevice, st_),
+                  "box items");
+        check(hipMemcpyAsync(flags_.get() + 7, &nBox, sizeof(int), hipMemcpyHostToDevice, st_), "box items");
+    }
     check(hipStreamSynchronize(st_), "rebuildActive");
     activeWork_ = off;
 }
@@ -499,14 +517,16 @@ bool Engine<T>::chainUsable(int itemSize) const {
 // rd_chain.hip's prefix and scatter after a histogram scan into labels.  Chains of at least
 // 2^kLongMinShift members are listed for the wave-summed sums, up to kLongWaves waves.
 template <typename T>
-void Engine<T>::enqueueChainOrder(int itemSize, const int* labels) {
+void Engine<T>::enqueueChainOrder(int itemSize, const int* labels, bool inc) {
     const EvolveSource es = evolveSource();
     const ChainArgs<T> ca{es.P, es.stride, es.index, dItems_.get(), compact() ? flags_.get() + 4 : nullptr,
                           dSegs_.get(), dSegK_.get(), dSegDone_.get(), (int)segs_.size(), labels, chainHist_.get(),
                           chainSegHistOff_.get(), chainSegKeyCap_.get(), chainSegRowOff_.get(), itemSize,
                           chainTotalRows_, chainTotals_.get(), sortedP_.get(), chainMStride_,
                           chainSegMemberOff_.get(), flags_.get(), chainOff_.get(), chainEnd_.get(), longList_.get(),
-                          chainLongCount_.get(), chainLongIdx_.get(), 1 << kLongMinShift, kLongWaves / dim_};
+                          chainLongCount_.get(), chainLongIdx_.get(), 1 << kLongMinShift, kLongWaves / dim_,
+                          inc ? chainPrefix_.get() : chainHist_.get(), inc ? touched_.get() : nullptr,
+                          inc ? act_.get() : nullptr, inc ? movedSlot_.get() : nullptr, incFirst_ ? 1 : 0};
     check(launch_chain_order<T>(ca, dim_, numItems_, chainKeyCapMax_, st_), "chain order");
 }
 
@@ -683,15 +703,33 @@ void Engine<T>::enqueueIteration(bool record, int slot, const IterLog* log, bool
     timers.chainPath = chainUsable(itemSize) ? 1 : 0;
     if (timers.chainPath) {
         // label histogram in the scan (one block per item in use), rd_chain.hip's prefix and
-        // scatter, then the ordered sums over the chain layout
+        // scatter, then the ordered sums over the chain layout; incremental iterations scan by
+        // boxes and look at the chains whose members changed only
+        const bool inc = incNow_ && !log && !record;
+        if (inc) {
+            const int* boxesInUse = compact() ? flags_.get() + 7 : nullptr;
+            const BoxScanArgs<T> ba{spQ_.get(), spStride_, spPerm_.get(), dBoxItems_.get(), boxesInUse, spBox_.get(),
+                                    spBound_.get(), S_.get(), Sold_.get(), sStride_, dSegs_.get(), dSegK_.get(),
+                                    dSegDone_.get(), dSegR1Sqr_.get(), flags_.get(), labS_.get(), labels,
+                                    movedSlot_.get(), touched_.get(), chainHist_.get(), chainSegHistOff_.get(),
+                                    itemSize};
+            timers.screenForm = 0;
+            check(launch_box_scan<T>(ba, dim_, (int)boxItems_.size(), incFirst_, st_), "box_scan");
+            if (incFirst_)
+                check(launch_label_hist(dItems_.get(), compact() ? flags_.get() + 4 : nullptr, numItems_, dSegs_.get(),
+                                        dSegK_.get(), dSegDone_.get(), labels, chainHist_.get(),
+                                        chainSegHistOff_.get(), itemSize, flags_.get(), st_),
+                      "label_hist");
+        } else {
         ScanArgs<T> sa{es.P, es.stride, es.index, S_.get(), sStride_, dItems_.get(), dSegs_.get(), dSegK_.get(),
                        dSegDone_.get(), dSegR1Sqr_.get(), flags_.get(), labels, flags_.get() + 3,
                        nullptr, nullptr, compact() ? flags_.get() + 4 : nullptr, nullptr, chainHist_.get(),
                        chainSegHistOff_.get(), chainSegKeyCap_.get(), itemSize};
         prepScreen(sa, screenForm());
         check(launch_evolve_scan<T>(sa, dim_, numItems_, options.ppt, options.scanThreads, 0, st_), "evolve_scan");
+        }
         if (ev) check(hipEventRecord(events_[3 * slot + 1], st_), "event");
-        enqueueChainOrder(itemSize, labels);
+        enqueueChainOrder(itemSize, labels, inc);
         // rows over the live slots of the evolve call (batches), else every slot below the bound
         const bool rowsValid = rowSlotsVersion_ == version_ && numRowSlots_ > 0;
         ShiftArgs<T> ha{es.P, es.stride, es.index, S_.get(), sStride_,
@@ -706,6 +744,11 @@ void Engine<T>::enqueueIteration(bool record, int slot, const IterLog* log, bool
         ha.longIdx = chainLongIdx_.get();
         ha.longMin = 1 << kLongMinShift;
         ha.longCap = kLongWaves / dim_;
+        if (inc) {
+            ha.act = act_.get();
+            ha.movedSlot = movedSlot_.get();
+            ha.Sold = Sold_.get();
+        }
         // the convergence bookkeeping in a launch of its own, not in the sum launch's last
         // block: that form's device-scope fence and completion count in each of the launch's
         // ~2000 blocks cost ~100 us per iteration of a 322k-point cloud against ~5 us here
@@ -947,6 +990,118 @@ void Engine<T>::autotuneBatchScan() {
     timers.tuneMs += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
+// Spatial order of every segment's samples, their blocks and boxes (rd_spatial.hip).
+template <typename T>
+void Engine<T>::buildSpatial() {
+    if (spatialValid_) return;
+    const int ns = (int)segs_.size();
+    const EvolveSource es = evolveSource();
+    int segBits = 0;
+    while ((int64_t(1) << segBits) < ns) ++segBits;
+    int maxP = 1;
+    for (const SegDesc& sd : segs_) maxP = std::max(maxP, (int)sd.nP);
+    // about 64 samples a cell of the largest segment (the occupied cells hold several times that)
+    const int bits = std::max(4, std::min({kSpatialBitsMax, ilog2(maxP) - 4, 30 - segBits}));
+    std::vector<WorkItem> items;
+    std::vector<int> firstItem(ns + 1);
+    boxItems_.clear();
+    for (int s = 0; s < ns; ++s) {
+        firstItem[s] = (int)items.size();
+        const int n = segs_[s].nP;
+        for (int i = 0; i < n; i += kBoundsItem) items.push_back({s, i, std::min(n, i + kBoundsItem), 0});
+        for (int i = 0; i < n; i += kBoxSamples)
+            boxItems_.push_back({s, i, std::min(n, i + kBoxSamples), (int)boxItems_.size()});
+    }
+    firstItem[ns] = (int)items.size();
+    const int numKeys = ns << bits;
+    DevBuf<WorkItem> dItems;
+    DevBuf<int> dFirst;
+    DevBuf<T> partial;
+    DevBuf<SpatialMap<T>> maps;
+    DevBuf<int64_t> dCount;
+    dItems.reserve(std::max<size_t>(items.size(), 1));
+    dFirst.reserve(firstItem.size());
+    partial.reserve(std::max<size_t>(items.size(), 1) * 2 * dim_);
+    maps.reserve(ns);
+    dCount.reserve(1);
+    spStride_ = round_up(totalP_, 64);
+    spQ_.reserve((size_t)spStride_ * dim_);
+    spPerm_.reserve(totalP_);
+    labS_.reserve(totalP_);
+    spBox_.reserve(std::max<size_t>(boxItems_.size(), 1) * 2 * dim_);
+    spBound_.reserve(std::max<size_t>(boxItems_.size(), 1));
+    dBoxItems_.reserve(std::max<size_t>(boxItems_.size(), 1));
+    sortWs_.reserve(sort_workspace_bytes(totalP_, numKeys));
+    check(hipMemcpyAsync(dItems.get(), items.data(), sizeof(WorkItem) * items.size(), hipMemcpyHostToDevice, st_), "sp");
+    check(hipMemcpyAsync(dFirst.get(), firstItem.data(), sizeof(int) * firstItem.size(), hipMemcpyHostToDevice, st_),
+          "spatial");
+    check(hipMemcpyAsync(dBoxItems_.get(), boxItems_.data(), sizeof(WorkItem) * boxItems_.size(),
+                         hipMemcpyHostToDevice, st_),
+          "spatial");
+    check(hipMemcpyAsync(dCount.get(), &totalP_, sizeof(int64_t), hipMemcpyHostToDevice, st_), "spatial");
+    const SpatialBuild<T> b{es.P, es.stride, es.index, dSegs_.get(), ns, dItems.get(), (int)items.size(),
+                            dFirst.get(), partial.get(), maps.get(), bits, labS_.get()};
+    check(launch_spatial_keys<T>(b, dim_, st_), "spatial keys");
+    check(stable_sort_by_key(labS_.get(), nullptr, dCount.get(), totalP_, numKeys, keys_.get(), spPerm_.get(),
+                             dM_.get(), sortWs_.get(), st_),
+          "spatial sort");
+    check(launch_spatial_gather<T>(es.P, es.stride, es.index, spPerm_.get(), totalP_, dim_, spQ_.get(), spStride_, st_),
+          "spatial gather");
+    check(launch_spatial_boxes<T>(spQ_.get(), spStride_, dBoxItems_.get(), dSegs_.get(), (int)boxItems_.size(), dim_,
+                                  spBox_.get(), st_),
+          "spatial boxes");
+    check(hipStreamSynchronize(st_), "spatial");   // the build's buffers are released on return
+    spatialValid_ = true;
+}
+
+// Whether the coming iterations of an evolve call (iters of them, 0: to convergence) run
+// incrementally, and if so their state.
+template <typename T>
+bool Engine<T>::prepareIncremental(long long iters) {
+    incNow_ = incFirst_ = false;
+    const int ns = (int)segs_.size();
+    // forced scan shapes, screens, orderings and sums keep the scans they name
+    if (!options.autotune || options.screen != 2 || options.chain != 1 || options.tolerance || options.segmented ||
+        ns == 0)
+        return false;
+    int64_t next = 0;
+    for (const SegDesc& sd : segs_) {
+        if (sd.pOff != next) return false;   // positions without a segment have no place in the order
+        next += sd.nP;
+    }
+    if (next != totalP_ || evolveSource().index) return false;
+    ensureChainScratch();
+    if (!chainReady_ || chainMeanKeys_ < kIncMinKeys) return false;
+    if (!spatialValid_ && iters > 0 && iters < kIncMinIters) return false;
+    // scatter blocks: about one per CU or more, and no fewer samples than keys
+    int itemSize = totalP_ < 131072 ? 256 : totalP_ < 262144 ? 512 : 1024;
+    while (itemSize < 2048 && chainMeanKeys_ > itemSize) itemSize *= 2;
+    options.ppt = itemSize >= 1024 ? itemSize / 512 : itemSize / 256;
+    options.scanThreads = itemSize >= 1024 ? 512 : 256;
+    options.persistent = false;
+    if (itemsPer_ != itemSize) {
+        buildWorkItems();
+        if (ns > 1) orderItemsByCost();
+    }
+    if (!chainUsable(itemSize)) return false;
+    buildSpatial();
+    const size_t slots = (size_t)std::max<int64_t>(totalSlots_, 1);
+    touched_.reserve(slots);
+    act_.reserve(slots);
+    movedSlot_.reserve(slots);
+    Sold_.reserve((size_t)std::max<int64_t>(sStride_, 1) * dim_);
+    chainPrefix_.reserve(chainHist_.n);
+    if (!compact())   // (a batch uploads its active boxes)
+        check(hipMemcpyAsync(dBoxItems_.get(), boxItems_.data(), sizeof(WorkItem) * boxItems_.size(),
+                             hipMemcpyHostToDevice, st_),
+              "box items");
+    timers.scanPpt = options.ppt;
+    timers.scanThreads = options.scanThreads;
+    timers.scanPersistent = 0;
+    incNow_ = incFirst_ = true;
+    return true;
+}
+
 template <typename T>
 void Engine<T>::autotuneScan() {
     ensureChainScratch();
@@ -1079,12 +1234,21 @@ void Engine<T>::evolveFixed(long long iters) {
     int f[2] = {0, 0};
     check(hipMemcpyAsync(dSegDone_.get(), zeros.data(), sizeof(int) * ns, hipMemcpyHostToDevice, st_), "done");
     check(hipMemcpyAsync(flags_.get(), f, sizeof(int) * 2, hipMemcpyHostToDevice, st_), "flags");
-    autotuneScan();
+    if (!prepareIncremental(iters)) autotuneScan();
     if (compact()) rebuildActive(zeros);
     const int batch = std::max(1, options.itersPerSync);
     long long done = 0;
+    if (incNow_) {
+        enqueueIteration(false, options.profile ? 0 : -1);
+        incFirst_ = false;
+        if (options.profile) {
+            check(hipStreamSynchronize(st_), "evolveFixed");
+            readEvents(1);
+        }
+        done = 1;
+    }
     hipGraphExec_t exec = nullptr;
-    const bool useGraph = options.graph && !options.profile && iters >= batch &&
+    const bool useGraph = options.graph && !options.profile && iters - done >= batch &&
                           captureIterations(batch, false, 0, &exec);
     // no convergence check between batches: they are all enqueued and the stream is synchronised
     // once (per batch only when profiling, whose events are read back per batch)
@@ -1101,6 +1265,7 @@ void Engine<T>::evolveFixed(long long iters) {
         done += nb;
     }
     check(hipStreamSynchronize(st_), "evolveFixed");
+    incNow_ = false;
     addEvolveBytes(std::vector<int>(ns, (int)std::min<long long>(iters, 0x7fffffff)));
     timers.evolveIterations += iters;
     timers.evolveMs += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -1258,8 +1423,8 @@ long long Engine<T>::evolve(long long maxIter, const std::vector<char>& active) 
     check(hipMemcpyAsync(dSegDone_.get(), done.data(), sizeof(int) * ns, hipMemcpyHostToDevice, st_), "done");
     check(hipMemcpyAsync(dSegMoved_.get(), zeros.data(), sizeof(int) * ns, hipMemcpyHostToDevice, st_), "moved");
     check(hipMemcpyAsync(flags_.get(), f, sizeof(int) * 2, hipMemcpyHostToDevice, st_), "flags");
-    autotuneScan();
-    segmentedNow_ = chooseSegmented(done);
+    if (!prepareIncremental(maxIter)) autotuneScan();
+    segmentedNow_ = !incNow_ && chooseSegmented(done);
     if (segmentedNow_) {
         // the scan runs over every item (done segments' items return at once)
         check(hipMemcpyAsync(dItems_.get(), items_.data(), sizeof(WorkItem) * items_.size(), hipMemcpyHostToDevice, st_),
@@ -1272,6 +1437,14 @@ long long Engine<T>::evolve(long long maxIter, const std::vector<char>& active) 
     long long iters = 0;
     const int batch = std::max(1, options.itersPerSync);
     std::vector<int> doneNow(ns);
+    if (incNow_) {
+        enqueueIteration(false, options.profile ? 0 : -1, nullptr, true, capIter);
+        incFirst_ = false;
+        if (options.profile) {
+            check(hipStreamSynchronize(st_), "evolve");
+            readEvents(1);
+        }
+    }
     // the iterations after convergence in a batch return at once (device all-done flag)
     hipGraphExec_t exec = nullptr;
     bool useGraph = options.graph && !options.profile && captureIterations(batch, true, capIter, &exec);
@@ -1306,7 +1479,7 @@ long long Engine<T>::evolve(long long maxIter, const std::vector<char>& active) 
         addEvolveBytes(segIter);
     }
     iters = std::max<long long>(iters, localIters);
-    segmentedNow_ = false;
+    segmentedNow_ = incNow_ = false;
     lastEvolveIters = iters;
     timers.evolveIterations += iters;
     timers.evolveMs += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

@@ -9,6 +9,7 @@
 #include "rd_evolve.hpp"
 #include "rd_local.hpp"
 #include "rd_sort.hpp"
+#include "rd_spatial.hpp"
 #include "rd_vjp.hpp"
 
 #include <chrono>
@@ -272,6 +273,16 @@ private:
     bool chainReady_ = false;
     long long chainEpoch_ = -1, countsEpoch_ = 0;   // countsEpoch_: bumped when chosen counts change
     int itemsPer_ = 0;                              // samples per work item of buildWorkItems
+    // incremental iterations (rd_spatial.hip): the samples' spatial order, valid while points and
+    // segments stay (spatialValid_), and the state of one evolve call (incNow_)
+    bool spatialValid_ = false, incNow_ = false, incFirst_ = false;
+    DevBuf<T> spQ_, spBox_, spBound_, Sold_;
+    int64_t spStride_ = 0;
+    DevBuf<int> spPerm_, labS_, touched_, act_, movedSlot_, chainPrefix_;
+    DevBuf<WorkItem> dBoxItems_;
+    std::vector<WorkItem> boxItems_;
+    void buildSpatial();
+    bool prepareIncremental(long long iters);
     // expanded-form screen: table rows (dim + 1) x sStride_ and per-segment centre and bound
     // (rd_screen.hip), rebuilt before every scan that uses them; tunedForm_: the form the
     // autotuner picked
@@ -337,7 +348,7 @@ private:
     // sizes the rd_chain.hip scratch for the current segments and chosen counts (outside graph
     // capture); chainUsable: the next iteration may take that path
     void ensureChainScratch();
-    void enqueueChainOrder(int itemSize, const int* labels);
+    void enqueueChainOrder(int itemSize, const int* labels, bool inc = false);
     bool chainUsable(int itemSize) const;
     // the general member ordering: stable sort of the scan's keys over totalP positions (keys
     // below kb), member coordinates into sortedP_, chain ranges and the wave list; returns the

@@ -285,6 +285,7 @@ __device__ __forceinline__ void chain_sum_rows(const ShiftArgs<T>& a, int64_t bl
         const int o = a.chainOff[chain];
         const int ce = a.chainEnd[chain];
         const int li = a.longCount ? a.longIdx[chain] : 0;
+        if (a.act && !a.act[slot]) seg = -1;
         if (seg >= 0 && !a.segDone[seg] && (int)(slot - a.segs[seg].sOff) < a.segK[seg]) {
             off = o;
             cnt = ce - o;

@@ -106,6 +106,12 @@ struct ShiftArgs {
     const int* longIdx;
     int longMin;
     int longCap;
+    // optional (incremental iterations, rd_spatial.hip), per slot: act -- the chains to sum (the
+    // others' members, hence their sums and positions, are unchanged); movedSlot -- set where a
+    // coordinate moves; Sold -- the summed chains' chosen points before the shift
+    const int* act;
+    int* movedSlot;
+    T* Sold;
 };
 
 // Mean of a chain and the shift rule of rd/cpu/brute_force/evolve.hpp:129-179 for one
@@ -124,13 +130,19 @@ __device__ __forceinline__ void shift_coordinate(const ShiftArgs<T>& a, int d, i
         thr = thr * fc;
         thr = thr * eps;
         T& s = a.S[d * a.sStride + slot];
+        if (a.Sold) a.Sold[d * a.sStride + slot] = s;
         if (fabs(mc - s) > thr) {
             s = mc;
             moved = true;
         }
+    } else if (a.Sold) {
+        a.Sold[d * a.sStride + slot] = a.S[d * a.sStride + slot];
     }
     if (a.outMoved) a.outMoved[d * a.movedStride + slot] = moved ? 1 : 0;
-    if (moved) a.segMoved[seg] = 1;
+    if (moved) {
+        a.segMoved[seg] = 1;
+        if (a.movedSlot) a.movedSlot[slot] = 1;
+    }
 }
 
 // Per-segment iteration count and convergence after an iteration, and the batch's all-done
