@@ -67,11 +67,21 @@ __global__ __launch_bounds__(256) void key_prefix_kernel(ChainArgs<T> a) {
     if (*a.allDone) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) *a.longCount = 0;   // the scatter's long-chain list
     const int lane = lane_id();
-    const int row = blockIdx.x * 4 + threadIdx.x / kWave;
-    if (row >= a.totalRows) return;
-    const int s = row_segment(a.segRowOff, a.numSegs, row);
+    int row = blockIdx.x * 4 + threadIdx.x / kWave;
+    int s;
+    SegDesc sd;
+    if (a.rowSlots) {
+        if (row >= a.numRowSlots) return;
+        const int slot = a.rowSlots[row];
+        s = a.slotSeg[slot];
+        sd = a.segs[s];
+        row = a.segRowOff[s] + (int)(slot - sd.sOff);
+    } else {
+        if (row >= a.totalRows) return;
+        s = row_segment(a.segRowOff, a.numSegs, row);
+        sd = a.segs[s];
+    }
     const int k = row - a.segRowOff[s];
-    const SegDesc sd = a.segs[s];
     const int nb = (sd.nP + a.itemSize - 1) / a.itemSize;
     if (a.act) {
         // incremental: a chain whose members are the last iteration's keeps its total and is left
@@ -355,8 +365,9 @@ bool chain_iteration_supported(int dim, int itemSize, int64_t keyCapMax) {
 template <typename T>
 hipError_t launch_chain_order(const ChainArgs<T>& a, int dim, int numItems, int keyCapMax, hipStream_t st) {
     if (!chain_iteration_supported(dim, a.itemSize, keyCapMax)) return hipErrorInvalidValue;
-    if (numItems <= 0 || a.totalRows <= 0) return hipSuccess;
-    hipLaunchKernelGGL((key_prefix_kernel<T>), dim3((unsigned)((a.totalRows + 3) / 4)), dim3(256), 0, st, a);
+    if (numItems <= 0 || a.totalRows <= 0 || (a.rowSlots && a.numRowSlots <= 0)) return hipSuccess;
+    const int rows = a.rowSlots ? a.numRowSlots : a.totalRows;
+    hipLaunchKernelGGL((key_prefix_kernel<T>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, a);
     bool ok = false;
     RD_DISPATCH_DIM(dim, { ok = launch_chain_dim<T, DIM>(a, numItems, keyCapMax, st); });
     return ok ? hipGetLastError() : hipErrorInvalidValue;

@@ -68,6 +68,10 @@ struct ChainArgs {
     int* act;
     int* moved;
     int allTouched;
+    // optional: the slots the prefix pass visits (numRowSlots of them) instead of every row
+    const int* rowSlots;
+    const int* slotSeg;
+    int numRowSlots;
 };
 
 // Launches the per-key prefix and the member scatter after a histogram scan over numItems

@@ -23,7 +23,7 @@ namespace {
 constexpr int kChooseFewSegs = 256;        // one block per CU
 constexpr int kChooseLargeFew = 4096;
 constexpr int kChooseLargeMany = 32768;
-constexpr double kIncMinKeys = 48;   // chosen points per segment (mean over samples)
+constexpr double kIncMinKeys = 8;    // chosen points per segment (mean over samples)
 constexpr int kIncMinIters = 4;
 
 inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
@@ -328,6 +328,8 @@ void Engine<T>::rebuildActive(const std::vector<int>& segDone) {
     }
     check(hipStreamSynchronize(st_), "rebuildActive");
     activeWork_ = off;
+    activeItems_ = n;
+    activeBoxes_ = nBox;
 }
 
 template <typename T>
@@ -519,6 +521,8 @@ bool Engine<T>::chainUsable(int itemSize) const {
 template <typename T>
 void Engine<T>::enqueueChainOrder(int itemSize, const int* labels, bool inc) {
     const EvolveSource es = evolveSource();
+    // a batch visits the live slots of its active segments (prepareRows)
+    const bool listed = compact() && rowSlotsVersion_ == version_ && numRowSlots_ > 0;
     const ChainArgs<T> ca{es.P, es.stride, es.index, dItems_.get(), compact() ? flags_.get() + 4 : nullptr,
                           dSegs_.get(), dSegK_.get(), dSegDone_.get(), (int)segs_.size(), labels, chainHist_.get(),
                           chainSegHistOff_.get(), chainSegKeyCap_.get(), chainSegRowOff_.get(), itemSize,
@@ -526,8 +530,9 @@ void Engine<T>::enqueueChainOrder(int itemSize, const int* labels, bool inc) {
                           chainSegMemberOff_.get(), flags_.get(), chainOff_.get(), chainEnd_.get(), longList_.get(),
                           chainLongCount_.get(), chainLongIdx_.get(), 1 << kLongMinShift, kLongWaves / dim_,
                           inc ? chainPrefix_.get() : chainHist_.get(), inc ? touched_.get() : nullptr,
-                          inc ? act_.get() : nullptr, inc ? movedSlot_.get() : nullptr, incFirst_ ? 1 : 0};
-    check(launch_chain_order<T>(ca, dim_, numItems_, chainKeyCapMax_, st_), "chain order");
+                          inc ? act_.get() : nullptr, inc ? movedSlot_.get() : nullptr, incFirst_ ? 1 : 0,
+                          listed ? rowSlots_.get() : nullptr, dSlotSeg_.get(), (int)numRowSlots_};
+    check(launch_chain_order<T>(ca, dim_, itemsInUse(), chainKeyCapMax_, st_), "chain order");
 }
 
 template <typename T>
@@ -714,9 +719,10 @@ void Engine<T>::enqueueIteration(bool record, int slot, const IterLog* log, bool
                                     movedSlot_.get(), touched_.get(), chainHist_.get(), chainSegHistOff_.get(),
                                     itemSize};
             timers.screenForm = 0;
-            check(launch_box_scan<T>(ba, dim_, (int)boxItems_.size(), incFirst_, st_), "box_scan");
+            check(launch_box_scan<T>(ba, dim_, compact() ? activeBoxes_ : (int)boxItems_.size(), incFirst_, st_),
+                  "box_scan");
             if (incFirst_)
-                check(launch_label_hist(dItems_.get(), compact() ? flags_.get() + 4 : nullptr, numItems_, dSegs_.get(),
+                check(launch_label_hist(dItems_.get(), compact() ? flags_.get() + 4 : nullptr, itemsInUse(), dSegs_.get(),
                                         dSegK_.get(), dSegDone_.get(), labels, chainHist_.get(),
                                         chainSegHistOff_.get(), itemSize, flags_.get(), st_),
                       "label_hist");
@@ -726,7 +732,7 @@ void Engine<T>::enqueueIteration(bool record, int slot, const IterLog* log, bool
                        nullptr, nullptr, compact() ? flags_.get() + 4 : nullptr, nullptr, chainHist_.get(),
                        chainSegHistOff_.get(), chainSegKeyCap_.get(), itemSize};
         prepScreen(sa, screenForm());
-        check(launch_evolve_scan<T>(sa, dim_, numItems_, options.ppt, options.scanThreads, 0, st_), "evolve_scan");
+        check(launch_evolve_scan<T>(sa, dim_, itemsInUse(), options.ppt, options.scanThreads, 0, st_), "evolve_scan");
         }
         if (ev) check(hipEventRecord(events_[3 * slot + 1], st_), "event");
         enqueueChainOrder(itemSize, labels, inc);
@@ -1098,6 +1104,11 @@ bool Engine<T>::prepareIncremental(long long iters) {
     timers.scanPpt = options.ppt;
     timers.scanThreads = options.scanThreads;
     timers.scanPersistent = 0;
+    // The first iterations change most labels.  Counts of more than 32 MB leave the caches, and an
+    // atomic per change then costs more than counting every label again: of the 2M-point grouped
+    // 6-D tiling (167M positions) iterations 2 to 9 took 6.0 to 1.8 ms by changes, 1.5 ms by full
+    // scans; the 1M helix (1.8 MB of counts) takes 18 us either way.
+    incFull_ = (int64_t)chainHist_.n * 4 / std::max(1, itemSize / 128) > (int64_t(32) << 20) ? 8 : 1;
     incNow_ = incFirst_ = true;
     return true;
 }
@@ -1238,15 +1249,14 @@ void Engine<T>::evolveFixed(long long iters) {
     if (compact()) rebuildActive(zeros);
     const int batch = std::max(1, options.itersPerSync);
     long long done = 0;
-    if (incNow_) {
+    for (; incNow_ && done < std::min<long long>(incFull_, iters); ++done) {
         enqueueIteration(false, options.profile ? 0 : -1);
-        incFirst_ = false;
         if (options.profile) {
             check(hipStreamSynchronize(st_), "evolveFixed");
             readEvents(1);
         }
-        done = 1;
     }
+    incFirst_ = false;
     hipGraphExec_t exec = nullptr;
     const bool useGraph = options.graph && !options.profile && iters - done >= batch &&
                           captureIterations(batch, false, 0, &exec);
@@ -1437,14 +1447,14 @@ long long Engine<T>::evolve(long long maxIter, const std::vector<char>& active) 
     long long iters = 0;
     const int batch = std::max(1, options.itersPerSync);
     std::vector<int> doneNow(ns);
-    if (incNow_) {
+    for (int i = 0; incNow_ && i < incFull_; ++i) {
         enqueueIteration(false, options.profile ? 0 : -1, nullptr, true, capIter);
-        incFirst_ = false;
         if (options.profile) {
             check(hipStreamSynchronize(st_), "evolve");
             readEvents(1);
         }
     }
+    incFirst_ = false;
     // the iterations after convergence in a batch return at once (device all-done flag)
     hipGraphExec_t exec = nullptr;
     bool useGraph = options.graph && !options.profile && captureIterations(batch, true, capIter, &exec);

@@ -275,7 +275,8 @@ private:
     int itemsPer_ = 0;                              // samples per work item of buildWorkItems
     // incremental iterations (rd_spatial.hip): the samples' spatial order, valid while points and
     // segments stay (spatialValid_), and the state of one evolve call (incNow_)
-    bool spatialValid_ = false, incNow_ = false, incFirst_ = false;
+    bool spatialValid_ = false, incNow_ = false, incFirst_ = false;   // incFirst_: full iterations
+    int incFull_ = 1;                                                   // how many of them
     DevBuf<T> spQ_, spBox_, spBound_, Sold_;
     int64_t spStride_ = 0;
     DevBuf<int> spPerm_, labS_, touched_, act_, movedSlot_, chainPrefix_;
@@ -330,6 +331,8 @@ private:
     bool compact() const { return segs_.size() > 1; }
     DevBuf<int> cKeys_, cPos_;
     int64_t activeWork_ = 0;
+    int activeItems_ = 0, activeBoxes_ = 0;   // of the active list (launch grids; graphs are captured again with it)
+    int itemsInUse() const { return compact() ? activeItems_ : numItems_; }
     void rebuildActive(const std::vector<int>& segDone);
     int persistentBlocks_ = 0;
     int persistentBlocks();
