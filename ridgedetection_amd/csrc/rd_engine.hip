@@ -694,7 +694,7 @@ void Engine<T>::enqueueIteration(bool record, int slot, const IterLog* log, bool
         if (ev) check(hipEventRecord(events_[3 * slot + 1], st_), "event");
         LocalArgs<T> la{es.P, es.stride, es.index, S_.get(), sStride_, dSegs_.get(), dSegK_.get(),
                         dSegR1Sqr_.get(), nullptr, (int)segs_.size(), segKStride_, segChunk_, 0, 0, nullptr, nullptr,
-                        nullptr, labels_.get(), dSegDone_.get(), dSegMoved_.get(), flags_.get()};
+                        nullptr, labels_.get(), dSegDone_.get(), dSegMoved_.get(), flags_.get(), 0};
         check(launch_segment_sums<T>(la, dim_, (int)segs_.size(), st_), "segment_sums");
         if (finalize)
             check(launch_evolve_finalize((int)segs_.size(), dSegDone_.get(), dSegMoved_.get(), dSegIter_.get(),
@@ -1391,7 +1391,8 @@ int Engine<T>::evolveLocal(long long maxIter, std::vector<int>& done) {
                    std::min(std::max(maxP, 1), kLocalChunk), maxIter > 0 ? (int)std::min<long long>(maxIter, 0x7fffffff) : 0,
                    options.evolveGuard > 0 ? (int)std::min<long long>(options.evolveGuard, 0x7fffffff) : 0x7fffffff,
                    dSegIter_.get(), flags_.get() + 5, flags_.get() + 6,
-                   nullptr, nullptr, nullptr, nullptr};
+                   nullptr, nullptr, nullptr, nullptr,
+                   local_fits_lds(dim_, sizeof(T), (int)round_up(std::max(maxK, 1), kChosenTile), std::max(maxP, 1))};
     check(launch_local_evolve<T>(a, dim_, st_), "local_evolve");
     int res[2] = {0, 0};
     check(hipMemcpyAsync(res, flags_.get() + 5, sizeof(int) * 2, hipMemcpyDeviceToHost, st_), "local flags");

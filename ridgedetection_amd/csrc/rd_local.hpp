@@ -37,10 +37,14 @@ struct LocalArgs {
     const int* segDone;
     int* segMoved;
     const int* allDone;
+    int samplesInLds;       // 1: every listed segment has at most pCap samples and local_fits_lds
 };
 
 // LDS bytes the local evolve needs for chosen stride kStride and chunks of `chunk` samples.
 size_t local_lds_bytes(int dim, size_t valueBytes, int kStride, int chunk);
+
+// True when a segment of maxP samples and its chosen points (stride kStride) fit the LDS whole.
+bool local_fits_lds(int dim, size_t valueBytes, int kStride, int maxP);
 
 // Runs every listed segment's evolve to convergence (or maxIter iterations): the
 // reference's evolve loop (rd/cpu/brute_force/evolve.hpp:237-459) with every iteration's

@@ -19,7 +19,9 @@
 // mean of a chosen point near an axis) most lanes are dirty, and after two such tiles in a row the
 // caller gets the sum so far back and finishes it with four waves (block_speculative_sum).
 //
-// Bound: latency of one wave's dependent steps, SCANNED.
+// Bound: latency of one wave's dependent steps.  Cycles per value of a long list, one wave: 1.95
+// float and 3.9 double, against 8.75 and 14.2 for additions fed by lane reads and 6.25 and 22.8 for
+// additions fed from LDS.
 #pragma once
 
 #include "rd_common.hpp"
