@@ -92,17 +92,10 @@ __global__ __launch_bounds__(256) void gather_members_kernel(const T* __restrict
 constexpr int kRowPer = 16;
 constexpr int kRowTile = kRowPer * 16;
 
-template <typename T>
-struct WideOf;
-template <>
-struct WideOf<float> { using type = float4; static constexpr int n = 4; };
-template <>
-struct WideOf<double> { using type = double2; static constexpr int n = 2; };
-
-// LDS per wave: four row slices padded by one wide read each
+// LDS per wave: four row slices padded by one wide read each, or a long sum's staged half tile
 template <typename T>
 constexpr int wave_lds_elems() {
-    return 4 * (kRowTile + WideOf<T>::n);
+    return std::max(4 * (kRowTile + WideOf<T>::n), serial_lds_elems<T>());
 }
 
 // sum + v.x + v.y (+ v.z + v.w), in that order
@@ -115,13 +108,6 @@ __device__ __forceinline__ float add_wide(float sum, float4 v) {
 __device__ __forceinline__ double add_wide(double sum, double2 v) {
     sum = sum + v.x;
     return sum + v.y;
-}
-
-// orders a wave's LDS accesses (the slices are private to the wave)
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Serial sum src[0] + src[1] + ... + src[cnt - 1] by a row of 16 lanes (every lane of the wave
@@ -355,14 +341,14 @@ struct HoverLds {
 
 template <typename T, int DIM>
 __device__ __forceinline__ void chain_sum_waves(const ShiftArgs<T>& a, int64_t entry, int64_t entries,
-                                                HoverLds<T>& sh) {
+                                                T* waveLds, HoverLds<T>& sh) {
     if (threadIdx.x == 0) sh.n = 0;
     __syncthreads();
     ListedChain c;
     if (entry < entries && listed_chain(a, entry / DIM, c)) {
         const int d = (int)(entry % DIM);
         const PartialSum<T> p =
-            wave_serial_sum<T>(a.sortedP + (int64_t)d * a.mStride + c.off, c.cnt, kHoverMin);
+            wave_serial_sum<T>(a.sortedP + (int64_t)d * a.mStride + c.off, c.cnt, kHoverMin, waveLds);
         if (lane_id() == 0) {
             if (p.done >= c.cnt) {
                 shift_coordinate(a, d, c.slot, c.seg, c.cnt, p.sum);
@@ -423,7 +409,8 @@ __global__ __launch_bounds__(256) void chain_sum_shift_kernel(ShiftArgs<T> a, in
     } else if (a.tolerance) {
         chain_sum_quarters<T, DIM>(a, (int64_t)blockIdx.x - rowBlocks, quarter);
     } else {
-        chain_sum_waves<T, DIM>(a, ((int64_t)blockIdx.x - rowBlocks) * kParts + threadIdx.x / kWave, entries, hover);
+        chain_sum_waves<T, DIM>(a, ((int64_t)blockIdx.x - rowBlocks) * kParts + threadIdx.x / kWave, entries,
+                                tiles[threadIdx.x / kWave], hover);
     }
 }
 

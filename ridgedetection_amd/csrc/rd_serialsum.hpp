@@ -8,20 +8,27 @@
 // numbers that can be added in any order.
 //
 // A tile gives each lane consecutive values.  The running sums at every lane are first predicted by
-// a floating-point scan; they differ from the serial ones by less than (values of the tile) / 2 + 40
-// units of the largest of them, and G below is more than that.  A lane is clean when every predicted
-// running sum from its start to its end is at least G inside one binade and none of its values lies
-// between two whole numbers: then the serial running sums are inside that binade too, its unit is
-// theirs, and neighbouring clean lanes share it.  The sum then advances from one dirty lane to the
-// next by the whole-number steps of the clean lanes between them (a difference of an integer scan),
-// and a dirty lane's values are added one by one.  Sums of one sign are dirty where they cross a
-// power of two and at about one value in between; where a sum hovers around zero (the coordinate
-// mean of a chosen point near an axis) most lanes are dirty, and after two such tiles in a row the
-// caller gets the sum so far back and finishes it with four waves (block_speculative_sum).
+// a floating-point scan.  Every partial sum on the way is a difference of two running sums, so no
+// rounding exceeds a unit of the largest running sum, and the serial ones' half of one: the
+// predictions are off by less than 3/2 (values of the tile) + 100 units, and G below is more than
+// that.  A half lane adds its values one after the other to its predicted start, and also to the
+// number one unit above it, which has the other parity.  When every predicted running sum on the way
+// is at least G inside one binade, the serial ones are inside that binade too, and the half lane's
+// whole-number steps are those of the start that has the serial sum's parity.  A lane is clean when
+// both halves are inside and take the same steps from either start; neighbouring clean lanes share
+// their binade.  The sum advances from one dirty lane to the next by the steps of the clean lanes
+// between them (a difference of an integer scan); a dirty lane's halves inside a binade are advanced
+// by the steps of the right parity, the others' values are added one by one (every lane adds its own
+// to the sum so far, and the dirty one's result is taken).  Sums of one sign are dirty where they
+// cross a power of two and at about one tie in between; where a sum hovers around zero (the
+// coordinate mean of a chosen point near an axis) most lanes are dirty, and after two such tiles in
+// a row the caller gets the sum so far back and finishes it with four waves (block_speculative_sum).
 //
-// Bound: latency of one wave's dependent steps.  Cycles per value of a long list, one wave: 1.95
-// float and 3.9 double, against 8.75 and 14.2 for additions fed by lane reads and 6.25 and 22.8 for
-// additions fed from LDS.
+// Bound: latency of one wave's dependent steps, and of a dirty lane's (about 350 cycles each; the
+// first 2,000 values have five to ten).  Cycles per value of a list of 32,768 floats, one wave: 1.14,
+// against 8.75 for additions fed by lane reads and 6.25 for additions fed from LDS; 3.2 for one of
+// 2,048.  With half the values a tile, lone ties added one by one and a rint of every value: 1.63
+// and 3.0, and 420 cycles a dirty lane.
 #pragma once
 
 #include "rd_common.hpp"
@@ -34,12 +41,10 @@ template <>
 struct Binade<float> {
     using Bits = unsigned;
     using Int = int;
-    static constexpr int mant = 23, expMax = 255, expBias = 127, perLane = 16;
-    static constexpr float guard = 1.220703125e-4f;   // 2^-13: 1024 units, a tile has 1024 values
+    static constexpr int mant = 23, expMax = 255, expBias = 127, perHalf = 16;
+    static constexpr float guard = 4.8828125e-4f;   // 2^-11: 4096 units, a tile has 2048 values
     static __device__ __forceinline__ Bits bits(float v) { return __float_as_uint(v); }
     static __device__ __forceinline__ float value(Bits b) { return __uint_as_float(b); }
-    static __device__ __forceinline__ float round(float v) { return __builtin_rintf(v); }
-    static __device__ __forceinline__ Bits first_lane(Bits b) { return (Bits)__builtin_amdgcn_readfirstlane((int)b); }
     static __device__ __forceinline__ Int lane(Int v, int l) { return __builtin_amdgcn_readlane(v, l); }
     template <int kCtrl, int kRows>
     static __device__ __forceinline__ Int dpp(Int old, Int v) {   // old where the lane has no source
@@ -54,16 +59,10 @@ template <>
 struct Binade<double> {
     using Bits = unsigned long long;
     using Int = long long;
-    static constexpr int mant = 52, expMax = 2047, expBias = 1023, perLane = 8;
-    static constexpr double guard = 9.094947017729282e-13;   // 2^-40
+    static constexpr int mant = 52, expMax = 2047, expBias = 1023, perHalf = 8;
+    static constexpr double guard = 9.094947017729282e-13;   // 2^-40: 4096 units, a tile has 1024 values
     static __device__ __forceinline__ Bits bits(double v) { return (Bits)__double_as_longlong(v); }
     static __device__ __forceinline__ double value(Bits b) { return __longlong_as_double((long long)b); }
-    static __device__ __forceinline__ double round(double v) { return __builtin_rint(v); }
-    static __device__ __forceinline__ Bits first_lane(Bits b) {
-        const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(b & 0xffffffffULL));
-        const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(b >> 32));
-        return ((Bits)hi << 32) | lo;
-    }
     static __device__ __forceinline__ Int lane(Int v, int l) { return (Int)read_lane((uint64_t)v, l); }
     template <int kCtrl, int kRows>
     static __device__ __forceinline__ Int dpp(Int old, Int v) {
@@ -92,7 +91,28 @@ __device__ __forceinline__ V wave_scan(V v, V id, Op op) {
     return v;
 }
 
-constexpr int kSerialSlack = 16;
+// a 16-byte read
+template <typename T>
+struct WideOf;
+template <>
+struct WideOf<float> { using type = float4; static constexpr int n = 4; };
+template <>
+struct WideOf<double> { using type = double2; static constexpr int n = 2; };
+
+// orders a wave's LDS accesses to a part of its own
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+constexpr int kSerialSlack = 4;
+
+// LDS values wave_serial_sum takes: the values of half the wave's lanes, 16 bytes apart
+template <typename T>
+constexpr int serial_lds_elems() {
+    return kWave / 2 * (2 * Binade<T>::perHalf + 16 / (int)sizeof(T));
+}
 
 // A running sum: `sum` holds the values before `done`.
 template <typename T>
@@ -106,98 +126,135 @@ struct PartialSum {
 // read (not used).  A sum that hovers is handed back unfinished while at least `hoverMin` values
 // are left.
 template <typename T>
-__device__ __forceinline__ PartialSum<T> wave_serial_sum(const T* __restrict__ src, int cnt, int hoverMin) {
+__device__ __forceinline__ PartialSum<T> wave_serial_sum(const T* __restrict__ src, int cnt, int hoverMin, T* lds) {
     using B = Binade<T>;
     using Int = typename B::Int;
     using Bits = typename B::Bits;
-    constexpr int kPer = B::perLane, kTile = kPer * kWave;
-    static_assert(kPer <= kSerialSlack, "a lane's last chunk may start at the list's last value");
+    constexpr int kHalf = B::perHalf, kPer = 2 * kHalf, kTile = kPer * kWave;
+    constexpr int kVec = 16 / sizeof(T), kLoads = kPer / kVec;
+    static_assert(kVec <= kSerialSlack && kPer * sizeof(T) == 128, "a lane's values are one line");
     const int lane = lane_id();
     cnt = __builtin_amdgcn_readfirstlane(cnt);
-    struct __attribute__((packed, aligned(sizeof(T)))) Chunk {
-        T v[kPer];
+    struct __attribute__((packed, aligned(sizeof(T)))) Vec {
+        T v[kVec];
     };
-    // lane l: values kPer l .. kPer l + kPer - 1 of the tile, +0 past the end (adding it changes no
-    // sum: a sum that starts at +0 is never -0).  Every tile is loaded the same way, whole, so that
-    // the loads of the next one stay in flight while this one is summed.
-    const int lastChunk = cnt > 0 ? (cnt - 1) / kPer * kPer : 0;
-    auto load = [&](int t0, Chunk& c) {
-        c = *reinterpret_cast<const Chunk*>(src + min(t0 + lane * kPer, lastChunk));
+    // Loads are coalesced, 16 bytes a lane, and go through LDS to the lane that sums them, the first
+    // half of the lanes' values and then the second's.  Every tile is loaded the same way, whole, so
+    // that the loads of the next one stay in flight while this one is summed.
+    const int lastVec = cnt > 0 ? (cnt - 1) / kVec * kVec : 0;
+    T* const put = lds + (lane / kLoads) * (kPer + kVec) + lane % kLoads * kVec;
+    const T* const get = lds + lane % (kWave / 2) * (kPer + kVec);
+    auto load = [&](int t0, Vec* c) {
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k)
+            c[k] = *reinterpret_cast<const Vec*>(src + min(t0 + (k * kWave + lane) * kVec, lastVec));
     };
     T s = T(0);
     if (cnt <= 0) return {s, 0};
-    Chunk nxt;
+    constexpr Bits kExp = (Bits)B::expMax << B::mant;
+    auto unit_of = [](T v) { return B::value((B::bits(v) & kExp) - ((Bits)B::mant << B::mant)); };
+    Vec nxt[kLoads];
     load(0, nxt);
     int hover = 0;
     for (int t0 = 0; t0 < cnt; t0 += kTile) {
+        // lane l: values kPer l .. kPer l + kPer - 1 of the tile, +0 past the end (adding it changes no
+        // sum: a sum that starts at +0 is never -0)
         T x[kPer];
 #pragma unroll
-        for (int j = 0; j < kPer; ++j) x[j] = t0 + lane * kPer + j < cnt ? nxt.v[j] : T(0);
+        for (int half = 0; half < 2; ++half) {
+            wave_lds_sync();
+#pragma unroll
+            for (int k = 0; k < kLoads / 2; ++k)
+                *reinterpret_cast<typename WideOf<T>::type*>(put + k * (kWave / kLoads) * (kPer + kVec)) =
+                    __builtin_bit_cast(typename WideOf<T>::type, nxt[half * (kLoads / 2) + k]);
+            wave_lds_sync();
+            if (lane / (kWave / 2) == half) {
+#pragma unroll
+                for (int k = 0; k < kLoads; ++k) {
+                    const Vec v = __builtin_bit_cast(Vec, reinterpret_cast<const typename WideOf<T>::type*>(get)[k]);
+#pragma unroll
+                    for (int j = 0; j < kVec; ++j) x[k * kVec + j] = v.v[j];
+                }
+            }
+        }
+        if (t0 + kTile > cnt) {
+#pragma unroll
+            for (int j = 0; j < kPer; ++j) x[j] = t0 + lane * kPer + j < cnt ? x[j] : T(0);
+        }
         load(t0 + kTile, nxt);
-        // predicted running sums: extremes inside the lane, start of the lane, largest of the tile
-        T run = T(0), mn = T(0), mx = T(0);
+        // the predicted sum at the start of each half of the lane, and the half's running sums from
+        // there (their extremes) and from one unit higher
+        T run[2] = {x[0], x[kHalf]}, at[2], unit[2], c0[2], c1[2], lo[2], hi[2];
 #pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            run = run + x[j];
-            mn = fmin(mn, run);
-            mx = fmax(mx, run);
+        for (int j = 1; j < kHalf; ++j)
+            for (int h = 0; h < 2; ++h) run[h] = run[h] + x[h * kHalf + j];
+        const T both = run[0] + run[1];
+        at[0] = s + (wave_scan<T>(both, T(0), [](T a, T b) { return a + b; }) - both);
+        at[1] = at[0] + run[0];
+        for (int h = 0; h < 2; ++h) {
+            unit[h] = unit_of(at[h]);
+            c1[h] = at[h] + unit[h];
+            c0[h] = lo[h] = hi[h] = at[h];
         }
-        const T upTo = wave_scan<T>(run, T(0), [](T a, T b) { return a + b; });
-        const T at = s + (upTo - run);
-        const T lo = at + mn, hi = at + mx;
-        const T big = fmax(fabs(lo), fabs(hi));
-        const T most = B::value(B::first_lane(B::bits(
-            read_lane(wave_scan<T>(big, T(0), [](T a, T b) { return fmax(a, b); }), kWave - 1))));
-        const T g = B::guard * most;
-        // the lane's binade, if it has one (the sums' magnitudes between near and far)
-        const T near = fmin(fabs(lo), fabs(hi)) - g, far = big + g;
-        const int ex = (int)((B::bits(near) >> B::mant) & (Bits)B::expMax);
-        bool clean = lo * hi > T(0) && near > T(0) && (B::bits(near) >> B::mant) == (B::bits(far) >> B::mant) &&
-                     ex > B::mant && ex < B::expMax - 1 && fabs(run) < far;   // run: no NaN on the way
-        const T inv = B::value((Bits)(2 * B::expBias + B::mant - (clean ? ex : B::expBias)) << B::mant);
-        T step = T(0), half = T(0);
 #pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            const T f = x[j] * inv;
-            const T r = B::round(f);
-            half = fmax(half, fabs(f - r));
-            step = step + r;
+        for (int j = 0; j < kHalf; ++j)
+            for (int h = 0; h < 2; ++h) {
+                c0[h] = c0[h] + x[h * kHalf + j];
+                c1[h] = c1[h] + x[h * kHalf + j];
+                lo[h] = fmin(lo[h], c0[h]);
+                hi[h] = fmax(hi[h], c0[h]);
+            }
+        T big[2];
+        for (int h = 0; h < 2; ++h) big[h] = fmax(fabs(lo[h]), fabs(hi[h]));
+        const T most = fmax(big[0], big[1]);
+        const T g = B::guard * read_lane(wave_scan<T>(most, T(0), [](T a, T b) { return fmax(a, b); }), kWave - 1);
+        bool inside[2], clean[2];
+        Int up0[2], up1[2];
+        for (int h = 0; h < 2; ++h) {
+            // the sums' magnitudes between near and far lie in one binade
+            const T near = fmin(fabs(lo[h]), fabs(hi[h])) - g, far = big[h] + g;
+            const int ex = (int)((B::bits(near) >> B::mant) & (Bits)B::expMax);
+            inside[h] = lo[h] * hi[h] > T(0) && near > T(0) && (B::bits(near) >> B::mant) == (B::bits(far) >> B::mant) &&
+                        ex > B::mant && ex < B::expMax - 1;
+            // units the magnitude grows by, counted by the bits of the one binade
+            up0[h] = (Int)(B::bits(c0[h]) - B::bits(at[h]));
+            up1[h] = (Int)(B::bits(c1[h]) - B::bits(at[h] + unit[h]));
+            clean[h] = inside[h] && up0[h] == up1[h];
         }
-        clean = clean && half < T(0.5);
-        const Int own = clean ? (Int)step : 0;
-        const Int steps = wave_scan<T>(own, Int(0), [](Int a, Int b) { return a + b; });
+        const Int steps = wave_scan<T>(clean[0] && clean[1] ? up0[0] + up0[1] : Int(0), Int(0),
+                                       [](Int a, Int b) { return a + b; });
         const int lanes = min(kWave, (cnt - t0 + kPer - 1) / kPer);
-        uint64_t dirty = __ballot(!clean && lane < lanes);
-        if (s == T(0) && __ballot(!(big == T(0))) == 0) dirty = 0;   // zeros leave a sum of zero
+        const uint64_t in0 = __ballot(inside[0]), in1 = __ballot(inside[1]);
+        uint64_t dirty = __ballot(!(clean[0] && clean[1]) && lane < lanes);
+        if (s == T(0) && __ballot(!(most == T(0))) == 0) dirty = 0;   // zeros leave a sum of zero
         if (__popcll(dirty) > kWave / 2) {
             if (++hover >= 2 && cnt - t0 >= hoverMin) return {s, t0};
         } else {
             hover = 0;
         }
+        auto advance = [](T from, Int by) { return B::value(B::bits(from) + (Bits)by); };   // in one binade
         Int before = 0;   // steps taken so far
         int from = 0;     // lanes in s
         for (;;) {
             const int to = dirty ? __builtin_ctzll(dirty) : lanes;
             if (to > from) {
                 const Int upto = B::lane(steps, to - 1);
-                if (upto != before) {
-                    const Bits sb = B::first_lane(B::bits(s));
-                    constexpr Bits kMant = ((Bits)1 << B::mant) - 1;
-                    const Bits signBit = (Bits)1 << (8 * sizeof(T) - 1);
-                    const Int m = (Int)((sb & kMant) | ((Bits)1 << B::mant));
-                    // x / U carries the sign of x: a negative sum's magnitude falls by it
-                    const Int now = (sb & signBit) ? m - (upto - before) : m + (upto - before);
-                    const Bits ue = ((sb & ~signBit) >> B::mant) - B::mant;
-                    s = (T)now * B::value((ue << B::mant) | (sb & signBit));
-                }
+                if (upto != before) s = advance(s, upto - before);
                 before = upto;
             }
             if (!dirty) break;
-            T v[kPer];
+            T v = s;   // every lane takes its own values; lane `to` started from the right sum
 #pragma unroll
-            for (int j = 0; j < kPer; ++j) v[j] = read_lane(x[j], to);
+            for (int h = 0; h < 2; ++h) {
+                if (((h ? in1 : in0) >> to) & 1) {
+                    // what a tie rounds to follows from the start's parity
+                    v = advance(v, (B::bits(v) ^ B::bits(at[h])) & 1 ? up1[h] : up0[h]);
+                } else {
 #pragma unroll
-            for (int j = 0; j < kPer; ++j) s = s + v[j];
+                    for (int j = 0; j < kHalf; ++j) v = v + x[h * kHalf + j];
+                }
+            }
+            s = read_lane(v, to);
             from = to + 1;
             dirty &= dirty - 1;
         }

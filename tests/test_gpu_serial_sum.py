@@ -2,7 +2,7 @@
 parallel binade by binade): sums, counts and the evolved points of one iteration against the
 oracle's serial sums, bit for bit, for values that cross binades back and forth, land exactly
 between two representable sums, stay on a power of two, cancel, or are tiny, at lengths around the
-512-value tiles and the length from which a chain is summed by a wave."""
+1024- and 2048-value tiles and the length from which a chain is summed by a wave."""
 
 import numpy as np
 import pytest
@@ -36,7 +36,7 @@ def _values(kind, n, g, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
-@pytest.mark.parametrize("n", [1024, 1025, 1535, 1536, 1537, 4099, 40001])
+@pytest.mark.parametrize("n", [1024, 1025, 1537, 2047, 2048, 2049, 4099, 40001])
 def test_one_chain_of_every_kind(oracle, n, dtype):
     from ridgedetection_amd._lib import Context
     g = np.random.Generator(np.random.PCG64(n))
