@@ -19,6 +19,7 @@
 // This replaces the histogram pass, the two-kernel histogram scan, the sort's scatter and the
 // chain-range pass of the general path (rd_sort.hip + chain bounds) for this case.
 #include "rd_chain.hpp"
+#include "rd_evolve.hpp"
 
 #include <algorithm>
 
@@ -83,13 +84,16 @@ __global__ __launch_bounds__(256) void key_prefix_kernel(ChainArgs<T> a) {
     }
     const int k = row - a.segRowOff[s];
     const int nb = (sd.nP + a.itemSize - 1) / a.itemSize;
+    bool segDone = a.segDone[s] != 0;
+    if (a.pendingMoved)
+        segDone = segDone || segment_converged(a.pendingMoved[s], a.pendingIter[s] + 1, a.maxIter);
     if (a.act) {
         // incremental: a chain whose members are the last iteration's keeps its total and is left
         // out of this iteration's ordering and sums
         const int64_t slot = sd.sOff + k;
-        const bool live = !a.segDone[s] && k < min(a.segK[s], a.segKeyCap[s]);
+        const bool live = !segDone && k < min(a.segK[s], a.segKeyCap[s]);
         const int t = live && (a.allTouched || a.touched[slot]) ? 1 : 0;
-        if (lane == 0 && live) {
+        if (lane == 0) {
             a.act[slot] = t;
             a.touched[slot] = 0;
             a.moved[slot] = 0;
@@ -111,7 +115,7 @@ __global__ __launch_bounds__(256) void key_prefix_kernel(ChainArgs<T> a) {
         }
         // rows of converged segments and of keys past the live count hold stale counts: loaded
         // (in bounds, in parallel with the flags' loads) but neither rewritten nor totalled
-        if (a.segDone[s] || k >= min(a.segK[s], a.segKeyCap[s])) {
+        if (segDone || k >= min(a.segK[s], a.segKeyCap[s])) {
             if (lane == 0) a.totals[row] = 0;
             return;
         }
@@ -154,7 +158,14 @@ __global__ __launch_bounds__(W * kWave) void member_scatter_kernel(ChainArgs<T> 
     int* lbase = gb + keyCap;
     int* wsum = lbase + keyCap;
     if (*a.allDone) return;
-    const int nItems = a.numItemsDev ? *a.numItemsDev : (int)gridDim.x;
+    if (a.pendingMoved && blockIdx.x == gridDim.x - 1) {
+        // the other blocks need no answer from here: a segment done by now has no chain to order
+        finalize_segments(a.numSegs, a.pendingDone, a.pendingMoved, a.pendingIter, a.maxIter, a.pendingAllDone,
+                          a.pendingTotal);
+        return;
+    }
+    const int nBlocks = (int)gridDim.x - (a.pendingMoved ? 1 : 0);
+    const int nItems = a.numItemsDev ? *a.numItemsDev : nBlocks;
     if ((int)blockIdx.x >= nItems) return;
     const WorkItem it = a.items[xcd_item(blockIdx.x, nItems)];
     const int s = it.seg;
@@ -340,8 +351,8 @@ void launch_scatter(const ChainArgs<T>& a, int numItems, int keyCap, hipStream_t
     constexpr int kStage = E + E * (int)(sizeof(T) / sizeof(int));
     const int region = std::max(W * keyCap, kStage);
     const size_t lds = sizeof(int) * ((size_t)region + 2 * (size_t)keyCap + W);
-    hipLaunchKernelGGL((member_scatter_kernel<T, DIM, W, C>), dim3((unsigned)numItems), dim3(W * kWave), lds, st, a,
-                       keyCap);
+    hipLaunchKernelGGL((member_scatter_kernel<T, DIM, W, C>), dim3((unsigned)(numItems + (a.pendingMoved ? 1 : 0))),
+                       dim3(W * kWave), lds, st, a, keyCap);
 }
 
 template <typename T, int DIM>

@@ -72,6 +72,15 @@ struct ChainArgs {
     const int* rowSlots;
     const int* slotSeg;
     int numRowSlots;
+    // optional (incremental): the bookkeeping of the iteration before (finalize_segments of
+    // rd_evolve.hpp), which has not run yet.  The prefix pass already leaves out the segments it
+    // will find done, and the scatter's last block runs it.
+    int* pendingMoved;          // segMoved, or null
+    int* pendingIter;           // segIter
+    int* pendingDone;           // segDone
+    int maxIter;
+    int* pendingAllDone;
+    int* pendingTotal;
 };
 
 // Launches the per-key prefix and the member scatter after a histogram scan over numItems

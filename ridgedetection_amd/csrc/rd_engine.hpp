@@ -351,7 +351,7 @@ private:
     // sizes the rd_chain.hip scratch for the current segments and chosen counts (outside graph
     // capture); chainUsable: the next iteration may take that path
     void ensureChainScratch();
-    void enqueueChainOrder(int itemSize, const int* labels, bool inc = false);
+    void enqueueChainOrder(int itemSize, const int* labels, bool inc = false, bool pending = false, int capIter = 0);
     bool chainUsable(int itemSize) const;
     // the general member ordering: stable sort of the scan's keys over totalP positions (keys
     // below kb), member coordinates into sortedP_, chain ranges and the wave list; returns the
@@ -359,8 +359,10 @@ private:
     int enqueueSortOrder(const int* labels, int64_t totalP, int64_t kb);
     // finalize: also the per-segment convergence bookkeeping (iteration cap capIter)
     void autotuneBatchScan();
+    // pending: the previous iteration's bookkeeping runs inside this one (enqueueBatch)
     void enqueueIteration(bool record, int slot = -1, const IterLog* log = nullptr, bool finalize = false,
-                          int capIter = 0);
+                          int capIter = 0, bool pending = false);
+    void enqueueBatch(int batch, bool finalize, int capIter);
     // state of the last evolveForward
     struct Tape {
         long long iters = 0;

@@ -145,6 +145,11 @@ __device__ __forceinline__ void shift_coordinate(const ShiftArgs<T>& a, int d, i
     }
 }
 
+// Whether a segment is done after its iteration number `iter` (from 1), which moved a point or not.
+__device__ __forceinline__ bool segment_converged(int moved, int iter, int maxIter) {
+    return moved == 0 || (maxIter > 0 && iter >= maxIter);
+}
+
 // Per-segment iteration count and convergence after an iteration, and the batch's all-done
 // flag, by one block of any size.
 __device__ __forceinline__ void finalize_segments(int numSegs, int* __restrict__ segDone, int* __restrict__ segMoved,
@@ -158,7 +163,7 @@ __device__ __forceinline__ void finalize_segments(int numSegs, int* __restrict__
         if (segDone[s]) continue;
         int it = segIter[s] + 1;
         segIter[s] = it;
-        bool done = (segMoved[s] == 0) || (maxIter > 0 && it >= maxIter);
+        const bool done = segment_converged(segMoved[s], it, maxIter);
         segMoved[s] = 0;
         if (done) segDone[s] = 1; else ++mine;
     }

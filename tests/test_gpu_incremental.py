@@ -135,3 +135,27 @@ def test_tiles(oracle, alg):
         c.set_points(P)
         S = c.tiled(alg, 0.06, 0.12, 20000, [2, 2, 2])
     np.testing.assert_array_equal(S, oracle.tiled(alg, P, 0.06, 0.12, 20000, [2, 2, 2]))
+
+
+@pytest.mark.parametrize("per_sync", [1, 2, 8])
+def test_caps_around_launch_batches(oracle, per_sync):
+    """The bookkeeping of an iteration runs inside the next one of its launch batch: caps that end
+    on either side of a batch's first and last iteration, several segments that converge apart."""
+    from ridgedetection_amd._lib import OPT_ITERS_PER_SYNC
+    P = synth.spiral2d(6000, seed=9)
+    S0, _ = oracle.choose(P, 0.45)
+    clouds = [synth.spiral2d(n, seed=n) for n in (900, 6000, 2500)]
+    radii = [0.45, 0.5, 0.55]
+    for cap in (1, 2, 3, 7, 8, 9, 10, 16, 17, 18):
+        print(f"case incremental cap={cap} per_sync={per_sync}", flush=True)
+        with _ctx(2, np.float32) as c:
+            c.set_option(OPT_ITERS_PER_SYNC, per_sync)
+            c.set_points(P)
+            c.set_chosen(S0)
+            S, it = c.evolve(0.45, cap)
+            res = c.batch(clouds, radii, [2 * r for r in radii], max_evolve_iters=cap)
+        ref, rit = oracle.evolve(P, S0, 0.45, cap)
+        np.testing.assert_array_equal(S, ref)
+        assert it == rit
+        for got, cloud, r in zip(res, clouds, radii):
+            np.testing.assert_array_equal(got, oracle.ridge_detection(cloud, r, 2 * r, max_evolve_iter=cap)[0])
