@@ -740,25 +740,7 @@ int rdhip_evolve_iteration(rdhip_ctx* ctx, double r, int32_t* labels, int32_t* c
         using T = decltype(zero);
         if (!ctx->hasChosen) return fail(RDHIP_ERR_STATE, "no chosen points (call rdhip_choose first)");
         e.setRadii({(T)r}, {(T)r});
-        std::vector<int> lab, cnt;
-        std::vector<T> sm;
-        std::vector<unsigned short> mv;
-        int flag = e.evolveIteration(labels ? &lab : nullptr, counts ? &cnt : nullptr, sums ? &sm : nullptr,
-                                     moved ? &mv : nullptr);
-        const int64_t K = e.totalCount();
-        const int64_t n = e.numPoints();
-        if (labels)
-            for (int64_t i = 0; i < n; ++i) labels[i] = lab[i];
-        if (counts)
-            for (int64_t k = 0; k < K; ++k) counts[k] = cnt[k];
-        if (sums) {
-            T* out = static_cast<T*>(sums);
-            const int64_t stride = (int64_t)sm.size() / ctx->dim;
-            for (int64_t k = 0; k < K; ++k)
-                for (int d = 0; d < ctx->dim; ++d) out[k * ctx->dim + d] = sm[d * stride + k];
-        }
-        if (moved)
-            for (int64_t k = 0; k < K; ++k) moved[k] = mv[k];
+        const int flag = e.evolveIteration(labels, counts, static_cast<T*>(sums), moved);
         if (out_flag) *out_flag = flag;
         return RDHIP_OK;
     });

@@ -100,6 +100,14 @@ __global__ void gather_chosen_kernel(const T* __restrict__ S, int64_t sStride, c
 
 inline unsigned grid_for(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 16384)); }
 
+// the state of an evolve call for the host (Engine::polled_)
+__global__ void publish_kernel(const int* __restrict__ flags, const int* __restrict__ segDone, int numSegs,
+                               int* __restrict__ out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < 2) out[i] = flags[i];
+    if (i < numSegs) out[2 + i] = segDone[i];
+}
+
 // copies every segment's first `cnt` slots (coordinates and chosen indices) to a new layout
 template <typename T>
 __global__ void relayout_slots_kernel(const T* __restrict__ S, int64_t sStride, const int* __restrict__ idx,
@@ -129,6 +137,9 @@ template <typename T>
 Engine<T>::~Engine() {
     if (graphExec_) (void)hipGraphExecDestroy(graphExec_);
     for (auto ev : events_) (void)hipEventDestroy(ev);
+    for (auto ev : batchEvent_)
+        if (ev) (void)hipEventDestroy(ev);
+    if (polled_) (void)hipHostFree(polled_);
     if (decWs_.nbr) (void)hipFree(decWs_.nbr);
     if (decWs_.par) (void)hipFree(decWs_.par);
     if (decWs_.boxes) (void)hipFree(decWs_.boxes);
@@ -257,6 +268,7 @@ void Engine<T>::setSegments(const std::vector<SegDesc>& segs, const std::vector<
         check(hipMemcpyAsync(dSlotSeg_.get(), slotSeg.data(), sizeof(int) * totalSlots_, hipMemcpyHostToDevice, st_),
               "slots");
         std::vector<int> zeros(ns, 0);
+        countsValid_ = false;
         check(hipMemcpyAsync(dSegK_.get(), zeros.data(), sizeof(int) * ns, hipMemcpyHostToDevice, st_), "K");
     }
     buildWorkItems();
@@ -615,6 +627,7 @@ void Engine<T>::choose() {
     preparePositions();
     const EvolveSource es = evolveSource();
     ++version_;
+    countsValid_ = false;
     chosenFromPoints_ = true;
     auto t0 = std::chrono::steady_clock::now();
     // Large segments take the rounds of rd_choose.hip, the others one block each.  One block
@@ -1296,6 +1309,23 @@ void Engine<T>::enqueueBatch(int batch, bool finalize, int capIter) {
     for (int b = 0; b < batch; ++b)
         enqueueIteration(false, options.profile ? b : -1, nullptr, finalize && (!fold || b == batch - 1), capIter,
                          fold && b > 0);
+    if (!finalize) return;
+    const int ns = (int)segs_.size();
+    hipLaunchKernelGGL(publish_kernel, dim3(grid_for(std::max(ns, 2))), dim3(256), 0, st_, flags_.get(), dSegDone_.get(),
+                       ns, polled_);
+    check(hipGetLastError(), "publish");
+}
+
+template <typename T>
+void Engine<T>::reservePolled(size_t n) {
+    for (auto& ev : batchEvent_)
+        if (!ev) check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate");
+    if (n <= polledSize_) return;
+    if (polled_) (void)hipHostFree(polled_);
+    polled_ = nullptr;
+    polledSize_ = 0;
+    check(hipHostMalloc((void**)&polled_, sizeof(int) * n, hipHostMallocDefault), "hipHostMalloc");
+    polledSize_ = n;
 }
 
 // Captures `batch` iterations into a graph.  The engine keeps one executable graph: a new
@@ -1465,6 +1495,7 @@ long long Engine<T>::evolve(long long maxIter, const std::vector<char>& active) 
     long long iters = 0;
     const int batch = std::max(1, options.itersPerSync);
     std::vector<int> doneNow(ns);
+    reservePolled((size_t)ns + 2);
     for (int i = 0; incNow_ && i < incFull_; ++i) {
         enqueueIteration(false, options.profile ? 0 : -1, nullptr, true, capIter);
         if (options.profile) {
@@ -1476,31 +1507,52 @@ long long Engine<T>::evolve(long long maxIter, const std::vector<char>& active) 
     // the iterations after convergence in a batch return at once (device all-done flag)
     hipGraphExec_t exec = nullptr;
     bool useGraph = options.graph && !options.profile && captureIterations(batch, true, capIter, &exec);
-    for (;;) {
-        if (useGraph) {
+    // The host reads the batch's outcome from its own memory, which the batch's last kernel writes:
+    // copies of the flags left the GPU idle for 60 to 100 us between batches.  From the fifth batch
+    // on one more is enqueued before the outcome of the last is known, so that the GPU does not wait
+    // for the host; if that one turns out to be past convergence, its launches cost about what two
+    // or three such waits did.
+    constexpr long long kAheadFrom = 4;
+    long long launched = 0, ended = 0;
+    auto launch = [&] {
+        if (useGraph)
             check(hipGraphLaunch(exec, st_), "hipGraphLaunch");
-        } else {
+        else
             enqueueBatch(batch, true, capIter);
-        }
-        check(hipMemcpyAsync(f, flags_.get(), sizeof(int) * 2, hipMemcpyDeviceToHost, st_), "flags");
-        check(hipStreamSynchronize(st_), "evolve");
+        check(hipEventRecord(batchEvent_[launched & 1], st_), "event");
+        ++launched;
+    };
+    const volatile int* state = polled_;
+    for (;;) {
+        if (launched == ended) launch();
+        const bool ahead = launched > kAheadFrom && !options.profile &&
+                           (options.evolveGuard <= 0 || iters + 3 * batch < options.evolveGuard);
+        if (ahead && launched == ended + 1) launch();
+        check(hipEventSynchronize(batchEvent_[ended & 1]), "evolve");
+        ++ended;
         if (options.profile) readEvents(batch);
-        iters = f[1];
-        if (f[0]) break;
+        // (a batch in flight may already have written a later outcome: equally good)
+        iters = state[1];
+        if (state[0]) break;
         if (options.evolveGuard > 0 && iters >= options.evolveGuard) throw std::runtime_error(guardMessage());
         if (compact() && !segmentedNow_) {
             // shrink the active work list once half of it belongs to converged segments
-            check(hipMemcpy(doneNow.data(), dSegDone_.get(), sizeof(int) * ns, hipMemcpyDeviceToHost), "done");
             int64_t remaining = 0;
             for (const WorkItem& it : items_)
-                if (!doneNow[it.seg]) remaining += it.end - it.start;
+                if (!state[2 + it.seg]) remaining += it.end - it.start;
             if (2 * remaining <= activeWork_) {
+                check(hipStreamSynchronize(st_), "evolve");
+                ended = launched;
+                if (state[0]) break;
+                for (int s = 0; s < ns; ++s) doneNow[s] = state[2 + s];
                 rebuildActive(doneNow);
                 prepareRows(doneNow);
                 if (exec) useGraph = captureIterations(batch, true, capIter, &exec);
             }
         }
     }
+    check(hipStreamSynchronize(st_), "evolve");
+    iters = state[1];
     {
         std::vector<int> segIter(ns);
         check(hipMemcpy(segIter.data(), dSegIter_.get(), sizeof(int) * ns, hipMemcpyDeviceToHost), "iterations");
@@ -1515,8 +1567,7 @@ long long Engine<T>::evolve(long long maxIter, const std::vector<char>& active) 
 }
 
 template <typename T>
-int Engine<T>::evolveIteration(std::vector<int>* labels, std::vector<int>* counts, std::vector<T>* sums,
-                               std::vector<unsigned short>* moved) {
+int Engine<T>::evolveIteration(int* labels, int* counts, T* sums, unsigned short* moved) {
     ++version_;
     const int ns = (int)segs_.size();
     std::vector<int> zeros(ns, 0);
@@ -1530,34 +1581,41 @@ int Engine<T>::evolveIteration(std::vector<int>* labels, std::vector<int>* count
     ensureChainScratch();
     enqueueIteration(true);
     std::vector<int> moved0(ns);
+    const std::vector<int> K = countsHost();
+    const int64_t total = std::accumulate(K.begin(), K.end(), int64_t(0));
     check(hipMemcpyAsync(moved0.data(), dSegMoved_.get(), sizeof(int) * ns, hipMemcpyDeviceToHost, st_), "moved");
-    const int64_t totalP = segs_.empty() ? 0 : segs_.back().pOff + segs_.back().nP;
-    if (labels) {
-        labels->resize((size_t)totalP);
-        check(hipMemcpyAsync(labels->data(), labels_.get(), sizeof(int) * totalP, hipMemcpyDeviceToHost, st_), "labels");
-    }
-    if (counts) {
-        counts->resize((size_t)totalSlots_);
-        check(hipMemcpyAsync(counts->data(), counts_.get(), sizeof(int) * totalSlots_, hipMemcpyDeviceToHost, st_),
-              "counts");
-    }
-    if (sums) {
-        sums->resize((size_t)sStride_ * dim_);
-        check(hipMemcpyAsync(sums->data(), sums_.get(), sizeof(T) * sStride_ * dim_, hipMemcpyDeviceToHost, st_),
-              "sums");
+    if (labels)
+        check(hipMemcpyAsync(labels, labels_.get(), sizeof(int) * nPoints_, hipMemcpyDeviceToHost, st_), "labels");
+    if (counts && total > 0)
+        check(hipMemcpyAsync(counts, counts_.get(), sizeof(int) * total, hipMemcpyDeviceToHost, st_), "counts");
+    DevBuf<T> rows;
+    DevBuf<int64_t> dOff;
+    std::vector<int64_t> off(ns, 0);
+    if (sums && total > 0) {
+        for (int s = 1; s < ns; ++s) off[s] = off[s - 1] + K[s - 1];
+        dOff.reserve(ns);
+        check(hipMemcpyAsync(dOff.get(), off.data(), sizeof(int64_t) * ns, hipMemcpyHostToDevice, st_), "off");
+        rows.reserve((size_t)total * dim_);
+        hipLaunchKernelGGL((gather_chosen_kernel<T>), dim3(ns), dim3(256), 0, st_, sums_.get(), sStride_, dSegs_.get(),
+                           dSegK_.get(), dOff.get(), dim_, rows.get(), (int)LAYOUT_ROW_MAJOR, (int64_t)dim_);
+        check(hipGetLastError(), "sums");
+        check(hipMemcpyAsync(sums, rows.get(), sizeof(T) * total * dim_, hipMemcpyDeviceToHost, st_), "sums");
     }
     std::vector<unsigned char> mv;
-    if (moved) {
-        mv.resize((size_t)totalSlots_ * dim_);
-        check(hipMemcpyAsync(mv.data(), moved_.get(), (size_t)totalSlots_ * dim_, hipMemcpyDeviceToHost, st_), "moved");
+    if (moved && total > 0) {
+        mv.resize((size_t)total * dim_);
+        check(hipMemcpy2DAsync(mv.data(), (size_t)total, moved_.get(), (size_t)totalSlots_, (size_t)total, (size_t)dim_,
+                               hipMemcpyDeviceToHost, st_),
+              "moved");
     }
     check(hipStreamSynchronize(st_), "evolveIteration");
-    if (moved) {
-        moved->assign((size_t)totalSlots_, 0);
-        for (int d = 0; d < dim_; ++d)
-            for (int64_t k = 0; k < totalSlots_; ++k)
-                if (mv[(size_t)d * totalSlots_ + k]) (*moved)[k] |= (unsigned short)(1u << d);
-    }
+    if (moved)
+        for (int64_t k = 0; k < total; ++k) {
+            unsigned short bits = 0;
+            for (int d = 0; d < dim_; ++d)
+                if (mv[(size_t)d * total + k]) bits |= (unsigned short)(1u << d);
+            moved[k] = bits;
+        }
     int any = 0;
     for (int v : moved0) any |= v;
     return any;
@@ -1692,6 +1750,7 @@ void Engine<T>::decimate(bool noCopyRule, std::vector<unsigned char>* keep) {
     const int ns = (int)segs_.size();
     if (ns == 0) return;
     ++version_;
+    countsValid_ = false;
     auto t0 = std::chrono::steady_clock::now();
     const int ng = (int)groupBegin_.size();
     const int64_t slots = std::max<int64_t>(totalSlots_, 1);
@@ -1737,12 +1796,17 @@ void Engine<T>::decimate(bool noCopyRule, std::vector<unsigned char>* keep) {
 // ------------------------------------------------------------------------------------
 template <typename T>
 std::vector<int> Engine<T>::countsHost() {
-    std::vector<int> k(segs_.size());
-    if (!k.empty()) {
-        check(hipMemcpyAsync(k.data(), dSegK_.get(), sizeof(int) * k.size(), hipMemcpyDeviceToHost, st_), "K");
-        check(hipStreamSynchronize(st_), "K");
+    if (!countsValid_ || counts0_.size() != segs_.size()) {
+        counts0_.resize(segs_.size());
+        if (!counts0_.empty()) {
+            check(hipMemcpyAsync(counts0_.data(), dSegK_.get(), sizeof(int) * counts0_.size(), hipMemcpyDeviceToHost,
+                                 st_),
+                  "K");
+            check(hipStreamSynchronize(st_), "K");
+        }
+        countsValid_ = true;
     }
-    return k;
+    return counts0_;
 }
 
 template <typename T>
@@ -1862,6 +1926,7 @@ std::vector<int> Engine<T>::chosenIndicesHost(int seg) {
 template <typename T>
 void Engine<T>::setChosen(int seg, const T* S, int64_t K, int layout, int64_t stride, bool onDevice) {
     ++version_;
+    countsValid_ = false;
     chosenFromPoints_ = false;
     if (seg < 0 || seg >= (int)segs_.size()) throw std::invalid_argument("segment out of range");
     if (K < 0 || K > segs_[seg].sCap) throw std::invalid_argument("too many chosen points for the segment");

@@ -164,9 +164,10 @@ public:
     // Exactly `iters` evolve iterations on every segment, ignoring convergence (benchmarks,
     // frozen-membership forward passes).
     void evolveFixed(long long iters);
-    // One evolve iteration on all segments, recording labels/counts/sums/moved on host.
-    int evolveIteration(std::vector<int>* labels, std::vector<int>* counts, std::vector<T>* sums,
-                        std::vector<unsigned short>* moved);
+    // One evolve iteration on all segments, recorded into host arrays (each optional): a label per
+    // sample, and per chosen point its member count, coordinate sums (a row of dim values) and the
+    // bits of the coordinates that moved.
+    int evolveIteration(int* labels, int* counts, T* sums, unsigned short* moved);
     void decimate(bool noCopyRule, std::vector<unsigned char>* keep = nullptr);
 
     // -- differentiated evolve (one segment) ------------------------------------------
@@ -198,6 +199,7 @@ public:
     void ridgeDetectionMixed(const RunOptions& opt);
 
     // -- results -------------------------------------------------------------------
+    // chosen points per segment (read back once after each change)
     std::vector<int> countsHost();
     int64_t totalCount();
     // Chosen points of all segments in segment order, into `out` with `layout`.
@@ -272,6 +274,14 @@ private:
     double chainMeanKeys_ = 0;   // keys per segment, averaged over samples
     bool chainReady_ = false;
     long long chainEpoch_ = -1, countsEpoch_ = 0;   // countsEpoch_: bumped when chosen counts change
+    std::vector<int> counts0_;    // dSegK_ on the host, while countsValid_
+    bool countsValid_ = false;
+    // what the host reads between batches of evolve iterations, written by the device into host
+    // memory (enqueueBatch): [0] all done, [1] iterations, then the segments' done flags
+    int* polled_ = nullptr;
+    size_t polledSize_ = 0;
+    hipEvent_t batchEvent_[2] = {};
+    void reservePolled(size_t n);
     int itemsPer_ = 0;                              // samples per work item of buildWorkItems
     // incremental iterations (rd_spatial.hip): the samples' spatial order, valid while points and
     // segments stay (spatialValid_), and the state of one evolve call (incNow_)
