@@ -15,9 +15,10 @@
 //                  (uniform inner loop: the partner coordinates are scalar loads);
 //   3. fill     -- CSR list of the 2 r2 neighbours of every element, with a "within r2" bit;
 //   4. scan     -- groups below kDecRoundsMin elements: one wave per group walks the
-//                  elements in order, 64 at a time: the window's counters and CSR rows are
-//                  staged in LDS, decisions are uniform, and a removal decrements its
-//                  neighbours' counters (LDS for the window, device-scope atomics beyond it);
+//                  elements in order, 64 at a time, with the group's counters and CSR rows in
+//                  LDS; decisions are uniform, and a removal decrements its neighbours'
+//                  counters (a larger group that resumes here stages a window of 64 at a time
+//                  and uses device-scope atomics beyond it);
 //      rounds   -- larger groups, one pass at a time: element e's test depends only on
 //                  which of its earlier (lower-index) neighbours the pass removed, since
 //                  its later neighbours are still live when the walk reaches it.  So in
@@ -36,7 +37,9 @@
 namespace rdhip {
 
 namespace {
-constexpr int kRowCap = 8192;   // CSR entries a window stages in LDS
+constexpr int kRowCap = 8192;   // CSR entries staged in LDS
+constexpr int kScanElems = 2048;   // elements of a group that is walked in LDS
+constexpr int kScanRows = 22528;   // entries of its rows, two bytes each (64 KB of LDS in all)
 
 __device__ __forceinline__ int ld_acq(const int* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -316,13 +319,104 @@ __global__ __launch_bounds__(256) void dec_prov_copy_kernel(DecArgs a, const int
     for (int k = 0; k < cnt; ++k) a.nbr[o + k] = prov[e * kDecProv + k];
 }
 
+// The serial walk of a group of at most kScanElems elements, by one wave: counters (c1 in the low
+// half of a word, c2 in the high one), live flags, row offsets and, if they fit, all rows in LDS.
+// Lane l holds element l of a window of 64; the wave goes from one element that its counters condemn
+// to the next, so elements that stay cost nothing, and reads the window's counters again after each
+// removal, as the removed row has changed them.
+//
+// Bound: the latency of a removal, about five dependent LDS accesses (rows that do not fit are read
+// from memory).  A walk that looked at every element in turn and kept the counters outside the window
+// in memory took 47 us for 180 chosen points of a 2,000-sample spiral, this one 7; 133 and 71 us for
+// those of a 1M-sample helix; 197 and 96 us for the tiles of a 120,000-sample 4-D chain.
+struct ScanLds {
+    int c[kScanElems];
+    int off[kScanElems + 1];
+    unsigned short rows[kScanRows];   // element within the group, the "within r2" bit below it
+};
+__device__ __forceinline__ void scan_group(const DecArgs& a, int g, int o, int n, int cnt, bool fresh, ScanLds& sh) {
+    const int lane = lane_id();
+    constexpr int kWindows = kScanElems / kWave;
+    const int base = a.rowOff[o];
+    const bool all = a.rowOff[o + n] - base <= kScanRows;
+    uint64_t mine = 0;   // lane w: the live elements of window w
+    for (int w = 0; w * kWave < n; ++w) {
+        const int i = w * kWave + lane;
+        const bool in = i < n;
+        sh.c[i] = in ? ld_acq(&a.c1[o + i]) | ld_acq(&a.c2[o + i]) << 16 : 0;
+        if (in) sh.off[i] = a.rowOff[o + i] - base;
+        const uint64_t live = __ballot(in && (fresh || ld_acq(&a.alive[o + i])));
+        if (lane == w) mine = live;
+    }
+    if (lane == 0) sh.off[n] = a.rowOff[o + n] - base;
+    if (all)
+        for (int t = lane, end = a.rowOff[o + n] - base; t < end; t += kWave)
+            sh.rows[t] = (unsigned short)(a.nbr[base + t] - 2 * o);
+    static_assert(kWindows <= kWave, "a lane keeps a window's live elements");
+    __syncthreads();
+    int left = -1;
+    bool stop = false;
+    while (left != cnt && cnt > 3 && !stop) {
+        left = cnt;
+        for (int w = 0; w * kWave < n && !stop; ++w) {
+            uint64_t live = (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(mine >> 32), w) << 32 |
+                            (unsigned)__builtin_amdgcn_readlane((int)(unsigned)mine, w);
+            uint64_t ahead = live;   // live elements the walk has not passed
+            while (ahead) {
+                if (a.noCopyRule && cnt - 1 < 3) break;   // nothing may go any more
+                const int c = sh.c[w * kWave + lane];
+                const uint64_t go = __ballot((c & 0xffff) >= 4 || (c >> 16) < 3) & ahead;
+                if (!go) break;
+                const int q = __builtin_ctzll(go);
+                --cnt;
+                live &= ~(1ull << q);
+                ahead &= ~((2ull << q) - 1);
+                const int i = w * kWave + q, end = sh.off[i + 1];
+                for (int t = sh.off[i] + lane; t < end; t += kWave) {
+                    const int v = all ? sh.rows[t] : a.nbr[base + t] - 2 * o;
+                    atomicSub(&sh.c[v >> 1], v & 1 ? 0x10001 : 0x10000);
+                }
+                __syncthreads();
+                if (!a.noCopyRule && cnt < 3) {
+                    stop = true;
+                    break;
+                }
+            }
+            if (lane == w) mine = live;
+        }
+    }
+    for (int w = 0; w * kWave < n; ++w) {
+        const uint64_t live = (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(mine >> 32), w) << 32 |
+                              (unsigned)__builtin_amdgcn_readlane((int)(unsigned)mine, w);
+        const int i = w * kWave + lane;
+        if (i < n) st_rel(&a.alive[o + i], (int)(live >> lane & 1));
+    }
+    if (lane == 0) {
+        a.groupLeft[g] = cnt;
+        a.groupMode[g] = kDecDone;
+    }
+}
+
 __global__ __launch_bounds__(64) void dec_scan_kernel(DecArgs a) {
-    __shared__ int wc1[kWave], wc2[kWave], wal[kWave];
-    __shared__ int rows[kRowCap];
+    __shared__ union {
+        ScanLds small;
+        struct {
+            int wc1[kWave], wc2[kWave], wal[kWave];
+            int rows[kRowCap];
+        } window;
+    } sh;
     const int g = blockIdx.x;
     const int mode = a.groupMode[g];
     if (mode != kDecSerial && mode != kDecResume) return;
     const int o = a.groupOff[g], n = a.groupCnt[g];
+    if (n <= kScanElems) {
+        scan_group(a, g, o, n, mode == kDecSerial ? n : a.groupAlive[g], mode == kDecSerial, sh.small);
+        return;
+    }
+    int* const wc1 = sh.window.wc1;
+    int* const wc2 = sh.window.wc2;
+    int* const wal = sh.window.wal;
+    int* const rows = sh.window.rows;
     const int lane = lane_id();
     if (mode == kDecSerial)
         for (int e = o + lane; e < o + n; e += kWave) st_rel(&a.alive[e], 1);

@@ -51,3 +51,22 @@ def test_long_rows_of_many_groups(oracle, dim, dtype):
         res = c.batch([p for p, _, _ in clouds], [a for _, a, _ in clouds], [b for _, _, b in clouds])
     for (P, r1, r2), S in zip(clouds, res):
         np.testing.assert_array_equal(S, oracle.ridge_detection(P, r1, r2)[0])
+
+
+@pytest.mark.parametrize("rule", [0, 1])
+@pytest.mark.parametrize("n", [3, 4, 63, 64, 65, 129, 777, 2047])
+def test_walk_in_lds(oracle, n, rule):
+    """Groups below 2,048 elements are walked in LDS: the edges of its windows of 64, rows that fit
+    and (the dense set of 777 and 2,047) rows that do not, and sets that thin out to three points."""
+    from ridgedetection_amd._lib import Context
+    g = np.random.Generator(np.random.PCG64(n))
+    S = g.uniform(0.0, 1.0, (n, 3)).astype(np.float32)
+    for r2 in (0.02, 0.5 / n ** (1 / 3), 1.0 / n ** (1 / 3), 0.4, 3.0):
+        print(f"case walk n={n} rule={rule} r2={r2:.4f}", flush=True)
+        with Context(3, np.float32) as c:
+            c.set_points(S)
+            c.set_chosen(S)
+            got, keep = c.decimate(r2, rule=rule)
+        ref, rkept = oracle.decimate(S, r2, nocopy=rule == 1)
+        np.testing.assert_array_equal(got, ref)
+        np.testing.assert_array_equal(np.flatnonzero(keep), rkept)
