@@ -23,7 +23,11 @@ namespace {
 constexpr int kChooseFewSegs = 256;        // one block per CU
 constexpr int kChooseLargeFew = 4096;
 constexpr int kChooseLargeMany = 32768;
-constexpr double kIncMinKeys = 8;    // chosen points per segment (mean over samples)
+// Chosen points per segment (mean over samples) from which iterations run incrementally.  With fewer
+// almost every block of samples depends on every point: the extended tiling of a 1M-sample helix (2
+// to 3 per tile) scans in 16 instead of 18 us, but its samples' order by space costs the scatter 3 us
+// more.  From 48 on instead, a 2M-point grouped 6-D tiling took 307 ms instead of 257.
+constexpr double kIncMinKeys = 8;
 constexpr int kIncMinIters = 4;
 
 inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
@@ -1120,11 +1124,12 @@ bool Engine<T>::prepareIncremental(long long iters) {
     timers.scanPpt = options.ppt;
     timers.scanThreads = options.scanThreads;
     timers.scanPersistent = 0;
-    // The first iterations change most labels.  Counts of more than 32 MB leave the caches, and an
-    // atomic per change then costs more than counting every label again: of the 2M-point grouped
-    // 6-D tiling (167M positions) iterations 2 to 9 took 6.0 to 1.8 ms by changes, 1.5 ms by full
-    // scans; the 1M helix (1.8 MB of counts) takes 18 us either way.
-    incFull_ = (int64_t)chainHist_.n * 4 / std::max(1, itemSize / 128) > (int64_t(32) << 20) ? 8 : 1;
+    // The first iterations change most labels.  Counts of more than 4 MB leave an XCD's L2, and an
+    // atomic per change then costs more than counting every label again: of a 2M-point grouped 6-D
+    // tiling iterations 2 to 9 took 6.8 to 2.0 ms by changes and 1.6 ms by full scans (the whole
+    // ridge 218 against 209.5 ms); 128 mixed clouds and the 1M helix (1.8 MB) take the same either
+    // way.
+    incFull_ = (int64_t)chainHist_.n * 4 / std::max(1, itemSize / 128) > (int64_t(4) << 20) ? 8 : 1;
     incNow_ = incFirst_ = true;
     return true;
 }

@@ -159,3 +159,23 @@ def test_caps_around_launch_batches(oracle, per_sync):
         assert it == rit
         for got, cloud, r in zip(res, clouds, radii):
             np.testing.assert_array_equal(got, oracle.ridge_detection(cloud, r, 2 * r, max_evolve_iter=cap)[0])
+
+
+def test_large_count_tables():
+    """More than 4 MB of counts: eight full iterations come first."""
+    from ridgedetection_amd._lib import OPT_AUTOTUNE
+    P = synth.helix3d(700000, seed=21, sigma=0.03)
+    res = []
+    for auto in (1, 0):
+        with _ctx(3, np.float32) as c:
+            c.set_option(OPT_AUTOTUNE, auto)
+            c.set_points(P)
+            S0, _ = c.choose(0.08)
+            print(f"case incremental large counts K={len(S0)} autotune={auto}", flush=True)
+            assert 1600 < len(S0) <= 2048
+            c.evolve_fixed(0.08, 13)
+            res.append(c.points())
+            S, it = c.evolve(0.08, 21)
+            res.append(S)
+    np.testing.assert_array_equal(res[0], res[2])
+    np.testing.assert_array_equal(res[1], res[3])
