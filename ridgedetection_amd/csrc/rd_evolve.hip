@@ -22,7 +22,8 @@
 //      members; L adapts so that at most kLongWaves entries are needed), or listed by length,
 //      go to a wave each instead, in the same launch, which computes the same serial sum in
 //      parallel (rd_serialsum.hpp).
-//   5. evolve_finalize -- per-segment iteration count and convergence; global all-done.
+//   5. evolve_finalize -- per-segment iteration count and convergence; global all-done (between
+//      the incremental iterations of a launch batch the next scatter does it, rd_chain.hip).
 #include "rd_evolve.hpp"
 #include "rd_rowsum.hpp"
 #include "rd_serialsum.hpp"
@@ -276,7 +277,7 @@ __device__ __forceinline__ void chain_sum_rows(const ShiftArgs<T>& a, int64_t bl
             off = o;
             cnt = ce - o;
             // a chain holding a multiple of L (or, by length, one of the listed long chains) is
-            // summed by a block (chain_sum_parts)
+            // summed by a wave (chain_sum_waves)
             const int64_t s0 = off, e1 = (int64_t)off + cnt - 1;
             const bool waveSummed =
                 a.longCount ? (cnt >= a.longMin && li < a.longCap)
