@@ -132,7 +132,10 @@ enum rdhip_option {
                                       segments (clouds, tiles) does the same per (value type,
                                       dimension, log2 samples, log2 segments) class over nine
                                       (samples per lane x threads x persistent queue or not)
-                                      shapes.  Cached per process */
+                                      shapes.  Cached per process.  Iterations that run
+                                      incrementally (default options, at most 2048 and on average
+                                      at least 8 chosen points per segment) are not tuned; 0 keeps
+                                      every iteration a full scan */
     RDHIP_OPT_SEGMENTED = 10,      /* 1: a batch whose active segments all have at most 65536
                                       samples and 1024 chosen points iterates as a batch-wide scan
                                       plus one workgroup per segment for the member sort, ordered
@@ -162,8 +165,10 @@ enum rdhip_option {
                                       every segment (cloud, tile) has at most 2048 chosen points and
                                       the segments have fewer chosen points than a scan block has
                                       samples (on average), the scan counts the labels per block and
-                                      one scatter writes the members in chain order; 2: that path
-                                      whenever the 2048 limit allows; 0: the general stable sort.
+                                      one scatter writes the members in chain order, and iterations
+                                      run incrementally where the other options are the defaults;
+                                      2: that path whenever the 2048 limit allows, every iteration a
+                                      full scan; 0: the general stable sort.
                                       Same results either way */
     RDHIP_OPT_SCREEN = 17          /* how the evolve scan screens (sample, chosen point) pairs
                                       before its exact decision: 2 (default): the fastest form as
