@@ -157,19 +157,24 @@ __global__ __launch_bounds__(W * kWave) void member_scatter_kernel(ChainArgs<T> 
     int* gb = lds + region;
     int* lbase = gb + keyCap;
     int* wsum = lbase + keyCap;
-    if (*a.allDone) return;
-    if (a.pendingMoved && blockIdx.x == gridDim.x - 1) {
-        // the other blocks need no answer from here: a segment done by now has no chain to order
+    // The last block of a launch with pending bookkeeping stores allDone and segDone while the others
+    // read them, so waves of one block may see different values: none of them leaves by itself.
+    const bool folded = a.pendingMoved != nullptr;
+    bool skip = *a.allDone != 0;
+    if (skip && !folded) return;
+    if (folded && blockIdx.x == gridDim.x - 1) {
+        if (skip) return;   // this block stores the flag, behind its barriers
         finalize_segments(a.numSegs, a.pendingDone, a.pendingMoved, a.pendingIter, a.maxIter, a.pendingAllDone,
                           a.pendingTotal);
         return;
     }
-    const int nBlocks = (int)gridDim.x - (a.pendingMoved ? 1 : 0);
+    const int nBlocks = (int)gridDim.x - (folded ? 1 : 0);
     const int nItems = a.numItemsDev ? *a.numItemsDev : nBlocks;
     if ((int)blockIdx.x >= nItems) return;
     const WorkItem it = a.items[xcd_item(blockIdx.x, nItems)];
     const int s = it.seg;
-    if (a.segDone[s]) return;
+    skip = skip || a.segDone[s];
+    if (skip && !folded) return;
     const SegDesc sd = a.segs[s];
     const int K = min(min(a.segK[s], a.segKeyCap[s]), keyCap);
     const int col = it.start / a.itemSize;
@@ -188,7 +193,7 @@ __global__ __launch_bounds__(W * kWave) void member_scatter_kernel(ChainArgs<T> 
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         const int i = it.start + (wave * C + c) * kWave + lane;
-        lraw[c] = i < it.end ? lab[i] : -1;
+        lraw[c] = i < it.end && !skip ? lab[i] : -1;
     }
     if (a.act) {
         // incremental: members of the chains ordered this iteration only
@@ -198,8 +203,10 @@ __global__ __launch_bounds__(W * kWave) void member_scatter_kernel(ChainArgs<T> 
             if (lraw[c] >= 0 && !a.act[lraw[c]]) lraw[c] = -1;
             any = any || lraw[c] >= 0;
         }
-        // the segment's first block also writes the chain ranges
-        if (!__syncthreads_or(any) && col != 0) return;
+        // The segment's first block also writes the chain ranges.  Waves that disagree on `skip` go on
+        // together: the prefix pass found the segment done too, so none of its chains is in act, their
+        // totals are 0 and no member is written.
+        if (!__syncthreads_or(col == 0 ? !skip : any)) return;
     }
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -379,6 +386,7 @@ bool chain_iteration_supported(int dim, int itemSize, int64_t keyCapMax) {
 template <typename T>
 hipError_t launch_chain_order(const ChainArgs<T>& a, int dim, int numItems, int keyCapMax, hipStream_t st) {
     if (!chain_iteration_supported(dim, a.itemSize, keyCapMax)) return hipErrorInvalidValue;
+    if (a.pendingMoved && !a.act) return hipErrorInvalidValue;   // (member_scatter_kernel's joint exit)
     if (numItems <= 0 || a.totalRows <= 0 || (a.rowSlots && a.numRowSlots <= 0)) return hipSuccess;
     const int rows = a.rowSlots ? a.numRowSlots : a.totalRows;
     hipLaunchKernelGGL((key_prefix_kernel<T>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, a);

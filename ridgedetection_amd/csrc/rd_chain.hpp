@@ -74,7 +74,8 @@ struct ChainArgs {
     int numRowSlots;
     // optional (incremental): the bookkeeping of the iteration before (finalize_segments of
     // rd_evolve.hpp), which has not run yet.  The prefix pass already leaves out the segments it
-    // will find done, and the scatter's last block runs it.
+    // will find done, and the scatter's last block runs it, beside the blocks that read the flags it
+    // stores: those take no decision from them that a wave would not share with its block.
     int* pendingMoved;          // segMoved, or null
     int* pendingIter;           // segIter
     int* pendingDone;           // segDone
