@@ -222,7 +222,10 @@ __global__ __launch_bounds__(kChooseBlock) void choose_filter_kernel(ChooseArgs<
             for (int j = 0; j < kG; ++j) s[j][d] = Sb[d * ss + k + j];
 #pragma unroll
         for (int j = 0; j < kG; ++j) live = live && !(exact_sqdist<T, DIM>(p, s[j]) <= rSqr);
-        if (!__ballot(live)) break;
+        if (!__ballot(live)) {
+            k = K;   // all covered: nothing is left for the remainder either
+            break;
+        }
     }
     for (; k < K; ++k) {
         T s[DIM];
