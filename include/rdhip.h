@@ -297,6 +297,11 @@ int rdhip_set_option(rdhip_ctx* ctx, int option, int64_t value);
 int rdhip_get_count(rdhip_ctx* ctx, int64_t* out_count);
 int rdhip_get_points(rdhip_ctx* ctx, void* out, int layout, int64_t stride, int on_device);
 int rdhip_get_timers(rdhip_ctx* ctx, rdhip_timers* out);
+/* How the last evolve ran (either output may be NULL).  out_incremental: full iterations that began
+ * the incremental ones of the last batch-wide evolve (RDHIP_OPT_CHAIN), 0: all of its iterations
+ * were full; out_local_lds: segments whose samples the last evolve inside workgroups
+ * (RDHIP_OPT_LOCAL) kept in LDS, 0: it read them from memory. */
+int rdhip_evolve_path(rdhip_ctx* ctx, int64_t* out_incremental, int64_t* out_local_lds);
 
 /* ---- phase-level entry points on the whole cloud (parity tests, custom drivers) ---- */
 

@@ -34,6 +34,7 @@ EXPORTS = [
     "rdhip_set_distances", "rdhip_hausdorff", "rdhip_distance_stats", "rdhip_batch_ridge_detection_dims",
     "rdhip_generate", "rdhip_generate_points", "rdhip_batch_generate", "rdhip_batch_run",
     "rdhip_set_chosen_ex", "rdhip_ridge_detection_own", "rdhip_choose_noalloc",
+    "rdhip_evolve_path",
 ]
 TREE_LOCAL, TREE_GROUPED, TREE_EXTENDED = 0, 1, 2
 OPT_PPT, OPT_ITERS_PER_SYNC, OPT_PROFILE, OPT_PERSISTENT, OPT_GRAPH, OPT_LOCAL = 0, 1, 2, 3, 4, 5
@@ -79,6 +80,7 @@ def load(path: str = LIB_PATH) -> C.CDLL:
         "rdhip_get_count": (i32, [vp, C.POINTER(i64)]),
         "rdhip_get_points": (i32, [vp, vp, i32, i64, i32]),
         "rdhip_get_timers": (i32, [vp, C.POINTER(Timers)]),
+        "rdhip_evolve_path": (i32, [vp, C.POINTER(i64), C.POINTER(i64)]),
         "rdhip_choose": (i32, [vp, C.c_double, C.POINTER(i64), vp]),
         "rdhip_set_chosen": (i32, [vp, vp, i64, i32]),
         "rdhip_set_chosen_ex": (i32, [vp, vp, i64, i32, i64, i32]),
@@ -197,6 +199,13 @@ class Context:
         t = Timers()
         self._check(self.lib.rdhip_get_timers(self.h, C.byref(t)))
         return {f: getattr(t, f) for f, _ in Timers._fields_}
+
+    def evolve_path(self) -> dict:
+        """How the last evolve ran: full iterations that began its incremental ones (0: none were),
+        and segments that a workgroup kept in LDS."""
+        inc, lds = C.c_int64(), C.c_int64()
+        self._check(self.lib.rdhip_evolve_path(self.h, C.byref(inc), C.byref(lds)))
+        return {"incremental": inc.value, "local_lds": lds.value}
 
     # -- drivers -------------------------------------------------------------------
     def ridge_detection(self, r1, r2, max_evolve_iters=0):

@@ -514,6 +514,14 @@ int rdhip_get_timers(rdhip_ctx* ctx, rdhip_timers* out) {
     });
 }
 
+int rdhip_evolve_path(rdhip_ctx* ctx, int64_t* out_incremental, int64_t* out_local_lds) {
+    return withEngine(ctx, [&](auto& e, auto) -> int {
+        if (out_incremental) *out_incremental = e.timers.incremental;
+        if (out_local_lds) *out_local_lds = e.timers.localLds;
+        return RDHIP_OK;
+    });
+}
+
 int rdhip_build_tree(rdhip_ctx* ctx, int kind, double r1, int64_t max_tile_capacity, const int64_t* tiles_per_dim,
                      int64_t* out_leaves) {
     if (kind < RDHIP_TREE_LOCAL || kind > RDHIP_TREE_EXTENDED) return fail(RDHIP_ERR_INVALID, "unknown tree kind");

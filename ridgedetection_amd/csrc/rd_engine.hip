@@ -1267,6 +1267,7 @@ void Engine<T>::evolveFixed(long long iters) {
     check(hipMemcpyAsync(dSegDone_.get(), zeros.data(), sizeof(int) * ns, hipMemcpyHostToDevice, st_), "done");
     check(hipMemcpyAsync(flags_.get(), f, sizeof(int) * 2, hipMemcpyHostToDevice, st_), "flags");
     if (!prepareIncremental(iters)) autotuneScan();
+    timers.incremental = incNow_ ? incFull_ : 0;
     if (compact()) rebuildActive(zeros);
     const int batch = std::max(1, options.itersPerSync);
     long long done = 0;
@@ -1448,6 +1449,7 @@ int Engine<T>::evolveLocal(long long maxIter, std::vector<int>& done) {
                    dSegIter_.get(), flags_.get() + 5, flags_.get() + 6,
                    nullptr, nullptr, nullptr, nullptr,
                    local_fits_lds(dim_, sizeof(T), (int)round_up(std::max(maxK, 1), kChosenTile), std::max(maxP, 1))};
+    timers.localLds = a.samplesInLds ? a.count : 0;
     check(launch_local_evolve<T>(a, dim_, st_), "local_evolve");
     int res[2] = {0, 0};
     check(hipMemcpyAsync(res, flags_.get() + 5, sizeof(int) * 2, hipMemcpyDeviceToHost, st_), "local flags");
@@ -1490,6 +1492,7 @@ long long Engine<T>::evolve(long long maxIter, const std::vector<char>& active) 
     check(hipMemcpyAsync(dSegMoved_.get(), zeros.data(), sizeof(int) * ns, hipMemcpyHostToDevice, st_), "moved");
     check(hipMemcpyAsync(flags_.get(), f, sizeof(int) * 2, hipMemcpyHostToDevice, st_), "flags");
     if (!prepareIncremental(maxIter)) autotuneScan();
+    timers.incremental = incNow_ ? incFull_ : 0;
     segmentedNow_ = !incNow_ && chooseSegmented(done);
     if (segmentedNow_) {
         // the scan runs over every item (done segments' items return at once)

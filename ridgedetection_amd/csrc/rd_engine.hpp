@@ -79,6 +79,9 @@ struct Timers {
     int chainPath = 0;                  // the last iteration enqueued took the rd_chain.hip path
     int screenForm = 0;                 // screen of the last scan enqueued: 0 direct, 1 expanded,
                                         // 2 expanded on the matrix cores
+    int incremental = 0;                // full iterations that began the last evolve's incremental
+                                        // ones, 0: all of its iterations were full
+    int localLds = 0;                   // segments the last local evolve kept in LDS whole
     double tuneMs = 0;                  // time spent timing candidate shapes
 };
 
