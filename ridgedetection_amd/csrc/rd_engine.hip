@@ -495,7 +495,8 @@ void Engine<T>::ensureChainScratch() {
     chainSegHistOff_.reserve(ns);
     chainSegMemberOff_.reserve(ns + 1);
     chainTotalPos_.reserve(1);
-    chainHist_.reserve((size_t)std::max<int64_t>(h, 1));
+    chainTable_ = std::max<int64_t>(h, 1);
+    chainHist_.reserve((size_t)chainTable_);
     chainTotals_.reserve((size_t)rows);
     if (sortedP_.n < (size_t)(m * dim_) + kSerialSlack) sortedP_.reserve((size_t)(m * dim_) + kSerialSlack);
     const int64_t entries = kLongWaves;   // the length-based wave list (at most kLongWaves / dim used)
@@ -1116,7 +1117,7 @@ bool Engine<T>::prepareIncremental(long long iters) {
     act_.reserve(slots);
     movedSlot_.reserve(slots);
     Sold_.reserve((size_t)std::max<int64_t>(sStride_, 1) * dim_);
-    chainPrefix_.reserve(chainHist_.n);
+    chainPrefix_.reserve((size_t)chainTable_);
     if (!compact())   // (a batch uploads its active boxes)
         check(hipMemcpyAsync(dBoxItems_.get(), boxItems_.data(), sizeof(WorkItem) * boxItems_.size(),
                              hipMemcpyHostToDevice, st_),
@@ -1129,7 +1130,7 @@ bool Engine<T>::prepareIncremental(long long iters) {
     // tiling iterations 2 to 9 took 6.8 to 2.0 ms by changes and 1.6 ms by full scans (the whole
     // ridge 218 against 209.5 ms); 128 mixed clouds and the 1M helix (1.8 MB) take the same either
     // way.
-    incFull_ = (int64_t)chainHist_.n * 4 / std::max(1, itemSize / 128) > (int64_t(4) << 20) ? 8 : 1;
+    incFull_ = chainTable_ * 4 / std::max(1, itemSize / 128) > (int64_t(4) << 20) ? 8 : 1;
     incNow_ = incFirst_ = true;
     return true;
 }

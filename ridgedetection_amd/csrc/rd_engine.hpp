@@ -274,6 +274,7 @@ private:
     DevBuf<int64_t> chainSegHistOff_, chainSegMemberOff_, chainTotalPos_;
     int64_t chainMStride_ = 0;
     int chainTotalRows_ = 0, chainKeyCapMax_ = 0;
+    int64_t chainTable_ = 0;     // counts of the current tables with 128-sample columns
     double chainMeanKeys_ = 0;   // keys per segment, averaged over samples
     bool chainReady_ = false;
     long long chainEpoch_ = -1, countsEpoch_ = 0;   // countsEpoch_: bumped when chosen counts change

@@ -103,3 +103,19 @@ def test_guard_with_a_batch_in_flight(oracle, guard):
         S, it = c.evolve(0.45)
     np.testing.assert_array_equal(S, ref)
     assert it == iters
+
+
+def test_full_iterations_follow_the_current_count_table():
+    """A large chosen set (count tables over 4 MB) starts with eight full iterations; a small one on
+    the same context afterwards with one, as it would on a context of its own."""
+    from ridgedetection_amd._lib import Context
+    P = synth.helix3d(1200000, seed=21, sigma=0.03)
+    with Context(3, np.float32) as c:
+        c.set_points(P)
+        S0 = np.ascontiguousarray(c.choose(0.07)[0][:2000])
+        assert len(S0) == 2000   # x 586 columns of 2048 samples: 4.7 MB of counts
+        for S, full in ((S0, 8), (np.ascontiguousarray(S0[::8]), 1), (S0, 8)):
+            c.set_chosen(S)
+            c.evolve_fixed(0.08, 12)
+            print(f"case path K={len(S)} {c.evolve_path()}", flush=True)
+            assert c.evolve_path()["incremental"] == full
