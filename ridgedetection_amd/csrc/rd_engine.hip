@@ -1307,18 +1307,21 @@ void Engine<T>::evolveFixed(long long iters) {
     timers.evolveMs += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
-// `batch` iterations.  Incremental ones leave their bookkeeping to the next one's scatter, so that
+// `batch` iterations, the first `full` of them full ones that begin incremental iterations.
+// Incremental ones leave their bookkeeping to the next one's scatter, so that
 // only the last of a batch launches it by itself: with a launch for each, the ridge of the 1M-sample
 // helix took 17.6 ms instead of 17.0, of a 20,000-sample spiral 5.3 instead of 5.0, of 128 mixed
 // clouds 313 instead of 306.  In between, the scan sees a segment that
 // the last iteration found done as still running; none of its points moved (or the iteration limit
 // ended it), so its labels stay as they are, or are not used again.
 template <typename T>
-void Engine<T>::enqueueBatch(int batch, bool finalize, int capIter) {
+void Engine<T>::enqueueBatch(int batch, bool finalize, int capIter, int full) {
     const bool fold = finalize && incNow_ && !options.profile;
-    for (int b = 0; b < batch; ++b)
+    for (int b = 0; b < batch; ++b) {
+        incFirst_ = b < full;
         enqueueIteration(false, options.profile ? b : -1, nullptr, finalize && (!fold || b == batch - 1), capIter,
                          fold && b > 0);
+    }
     if (!finalize) return;
     const int ns = (int)segs_.size();
     hipLaunchKernelGGL(publish_kernel, dim3(grid_for(std::max(ns, 2))), dim3(256), 0, st_, flags_.get(), dSegDone_.get(),
@@ -1508,17 +1511,9 @@ long long Engine<T>::evolve(long long maxIter, const std::vector<char>& active) 
     const int batch = std::max(1, options.itersPerSync);
     std::vector<int> doneNow(ns);
     reservePolled((size_t)ns + 2);
-    for (int i = 0; incNow_ && i < incFull_; ++i) {
-        enqueueIteration(false, options.profile ? 0 : -1, nullptr, true, capIter);
-        if (options.profile) {
-            check(hipStreamSynchronize(st_), "evolve");
-            readEvents(1);
-        }
-    }
-    incFirst_ = false;
     // the iterations after convergence in a batch return at once (device all-done flag)
     hipGraphExec_t exec = nullptr;
-    bool useGraph = options.graph && !options.profile && captureIterations(batch, true, capIter, &exec);
+    bool useGraph = false;
     // The host reads the batch's outcome from its own memory, which the batch's last kernel writes:
     // copies of the flags left the GPU idle for 60 to 100 us between batches.  From the fifth batch
     // on one more is enqueued before the outcome of the last is known, so that the GPU does not wait
@@ -1526,15 +1521,19 @@ long long Engine<T>::evolve(long long maxIter, const std::vector<char>& active) 
     // or three such waits did.
     constexpr long long kAheadFrom = 4;
     long long launched = 0, ended = 0;
+    int full = incNow_ ? incFull_ : 0;   // full iterations to come: the first batches hold them
     auto launch = [&] {
-        if (useGraph)
+        if (full == 0 && useGraph)
             check(hipGraphLaunch(exec, st_), "hipGraphLaunch");
         else
-            enqueueBatch(batch, true, capIter);
+            enqueueBatch(batch, true, capIter, std::min(full, batch));
+        full -= std::min(full, batch);
         check(hipEventRecord(batchEvent_[launched & 1], st_), "event");
         ++launched;
     };
     const volatile int* state = polled_;
+    if (full > 0) launch();   // the GPU works while the graph is captured
+    useGraph = options.graph && !options.profile && captureIterations(batch, true, capIter, &exec);
     for (;;) {
         if (launched == ended) launch();
         const bool ahead = launched > kAheadFrom && !options.profile &&

@@ -376,7 +376,7 @@ private:
     // pending: the previous iteration's bookkeeping runs inside this one (enqueueBatch)
     void enqueueIteration(bool record, int slot = -1, const IterLog* log = nullptr, bool finalize = false,
                           int capIter = 0, bool pending = false);
-    void enqueueBatch(int batch, bool finalize, int capIter);
+    void enqueueBatch(int batch, bool finalize, int capIter, int full = 0);
     // state of the last evolveForward
     struct Tape {
         long long iters = 0;

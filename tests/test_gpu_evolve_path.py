@@ -119,3 +119,43 @@ def test_full_iterations_follow_the_current_count_table():
             c.evolve_fixed(0.08, 12)
             print(f"case path K={len(S)} {c.evolve_path()}", flush=True)
             assert c.evolve_path()["incremental"] == full
+
+
+@pytest.mark.parametrize("per_sync,guard", [(64, 64), (1, 1), (2, 3), (5, 16), (8, 8)])
+def test_guard_stops_after_whole_launch_batches(oracle, per_sync, guard):
+    """The iteration limit is looked at after every per_sync iterations from the first on."""
+    from ridgedetection_amd._lib import Context, OPT_EVOLVE_GUARD, OPT_ITERS_PER_SYNC, OPT_LOCAL, RDError
+    P = synth.spiral2d(20000, seed=4)
+    S0, _ = oracle.choose(P, 0.45)
+    _, iters = oracle.evolve(P, S0, 0.45)
+    assert iters == 65
+    ran = -(-guard // per_sync) * per_sync
+    print(f"case guard={guard} per_sync={per_sync} stops after {ran}", flush=True)
+    with Context(2, np.float32) as c:
+        c.set_option(OPT_LOCAL, 0)
+        c.set_option(OPT_ITERS_PER_SYNC, per_sync)
+        c.set_points(P)
+        c.set_chosen(S0)
+        c.set_option(OPT_EVOLVE_GUARD, guard)
+        with pytest.raises(RDError, match="iteration guard"):
+            c.evolve(0.45)
+        np.testing.assert_array_equal(c.points(), oracle.evolve(P, S0, 0.45, ran)[0])
+
+
+def test_guard_within_the_full_iterations():
+    """Eight full iterations first, stopped after three of them."""
+    from ridgedetection_amd._lib import Context, OPT_EVOLVE_GUARD, OPT_ITERS_PER_SYNC, RDError
+    P = synth.helix3d(1200000, seed=21, sigma=0.03)
+    with Context(3, np.float32) as c:
+        c.set_points(P)
+        S0 = np.ascontiguousarray(c.choose(0.07)[0][:2000])
+        c.set_chosen(S0)
+        want, _ = c.evolve(0.07, 3)
+        c.set_chosen(S0)
+        c.set_option(OPT_ITERS_PER_SYNC, 3)
+        c.set_option(OPT_EVOLVE_GUARD, 2)
+        print(f"case guard within {len(S0)} chosen points' full iterations", flush=True)
+        with pytest.raises(RDError, match="iteration guard"):
+            c.evolve(0.07)
+        assert c.evolve_path()["incremental"] == 8
+        np.testing.assert_array_equal(c.points(), want)
