@@ -28,7 +28,15 @@ constexpr int kChooseLargeMany = 32768;
 // to 3 per tile) scans in 16 instead of 18 us, but its samples' order by space costs the scatter 3 us
 // more.  From 48 on instead, a 2M-point grouped 6-D tiling took 307 ms instead of 257.
 constexpr double kIncMinKeys = 8;
+// Iterations from which the samples are put in order for them.  The order costs 0.1 to 0.25 ms, and
+// an iteration saves little where a full scan is short: evolve_fixed on new points, 3-D floats, full
+// against incremental at 4 and 7 iterations: 20,000 samples x 167 points 0.19 : 0.27 and 0.26 : 0.35
+// ms, 130,000 x 213 0.23 : 0.32 and 0.34 : 0.42, 300,000 x 250 0.31 : 0.35 and 0.49 : 0.46, 1M x 290
+// 0.60 : 0.51 and 0.97 : 0.68.  From 8 on, a launch batch, full ones also capture a graph (0.7 ms and
+// more at 20,000 samples against 0.36).
 constexpr int kIncMinIters = 4;
+constexpr int kIncMinItersSmall = 8;
+constexpr double kIncSmallPairs = 1 << 26;
 
 inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
@@ -1099,7 +1107,8 @@ bool Engine<T>::prepareIncremental(long long iters) {
     if (next != totalP_ || evolveSource().index) return false;
     ensureChainScratch();
     if (!chainReady_ || chainMeanKeys_ < kIncMinKeys) return false;
-    if (!spatialValid_ && iters > 0 && iters < kIncMinIters) return false;
+    const int minIters = (double)totalP_ * chainMeanKeys_ < kIncSmallPairs ? kIncMinItersSmall : kIncMinIters;
+    if (!spatialValid_ && iters > 0 && iters < minIters) return false;
     // scatter blocks: about one per CU or more, and no fewer samples than keys
     int itemSize = totalP_ < 131072 ? 256 : totalP_ < 262144 ? 512 : 1024;
     while (itemSize < 2048 && chainMeanKeys_ > itemSize) itemSize *= 2;

@@ -159,3 +159,22 @@ def test_guard_within_the_full_iterations():
             c.evolve(0.07)
         assert c.evolve_path()["incremental"] == 8
         np.testing.assert_array_equal(c.points(), want)
+
+
+def test_short_evolves_on_new_points(oracle):
+    """Ordering new samples by space pays from eight iterations on, or from four where a full scan
+    has 2^26 pairs or more; an order that is there is used."""
+    from ridgedetection_amd._lib import Context, OPT_LOCAL
+    for n, steps in ((20000, ((7, 0), (8, 1), (4, 1), (1, 1))), (400000, ((3, 0), (4, 1), (2, 1)))):
+        P = synth.helix3d(n, seed=4, sigma=0.04)
+        with Context(3, np.float32) as c:
+            c.set_option(OPT_LOCAL, 0)
+            c.set_points(P)
+            S0, _ = c.choose(0.2)
+            for iters, inc in steps:
+                c.set_chosen(S0)
+                c.evolve_fixed(0.2, iters)
+                print(f"case path n={n} K={len(S0)} iterations={iters} {c.evolve_path()}", flush=True)
+                assert c.evolve_path()["incremental"] == inc
+                if n < 100000:
+                    np.testing.assert_array_equal(c.points(), oracle.evolve(P, S0, 0.2, iters)[0])
