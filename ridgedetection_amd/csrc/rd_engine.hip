@@ -1049,16 +1049,11 @@ void Engine<T>::buildSpatial() {
     }
     firstItem[ns] = (int)items.size();
     const int numKeys = ns << bits;
-    DevBuf<WorkItem> dItems;
-    DevBuf<int> dFirst;
-    DevBuf<T> partial;
-    DevBuf<SpatialMap<T>> maps;
-    DevBuf<int64_t> dCount;
-    dItems.reserve(std::max<size_t>(items.size(), 1));
-    dFirst.reserve(firstItem.size());
-    partial.reserve(std::max<size_t>(items.size(), 1) * 2 * dim_);
-    maps.reserve(ns);
-    dCount.reserve(1);
+    spItems_.reserve(std::max<size_t>(items.size(), 1));
+    spFirst_.reserve(firstItem.size());
+    spPartial_.reserve(std::max<size_t>(items.size(), 1) * 2 * dim_);
+    spMaps_.reserve(ns);
+    spCount_.reserve(1);
     spStride_ = round_up(totalP_, 64);
     spQ_.reserve((size_t)spStride_ * dim_);
     spPerm_.reserve(totalP_);
@@ -1067,17 +1062,17 @@ void Engine<T>::buildSpatial() {
     spBound_.reserve(std::max<size_t>(boxItems_.size(), 1));
     dBoxItems_.reserve(std::max<size_t>(boxItems_.size(), 1));
     sortWs_.reserve(sort_workspace_bytes(totalP_, numKeys));
-    check(hipMemcpyAsync(dItems.get(), items.data(), sizeof(WorkItem) * items.size(), hipMemcpyHostToDevice, st_), "sp");
-    check(hipMemcpyAsync(dFirst.get(), firstItem.data(), sizeof(int) * firstItem.size(), hipMemcpyHostToDevice, st_),
+    check(hipMemcpyAsync(spItems_.get(), items.data(), sizeof(WorkItem) * items.size(), hipMemcpyHostToDevice, st_), "sp");
+    check(hipMemcpyAsync(spFirst_.get(), firstItem.data(), sizeof(int) * firstItem.size(), hipMemcpyHostToDevice, st_),
           "spatial");
     check(hipMemcpyAsync(dBoxItems_.get(), boxItems_.data(), sizeof(WorkItem) * boxItems_.size(),
                          hipMemcpyHostToDevice, st_),
           "spatial");
-    check(hipMemcpyAsync(dCount.get(), &totalP_, sizeof(int64_t), hipMemcpyHostToDevice, st_), "spatial");
-    const SpatialBuild<T> b{es.P, es.stride, es.index, dSegs_.get(), ns, dItems.get(), (int)items.size(),
-                            dFirst.get(), partial.get(), maps.get(), bits, labS_.get()};
+    check(hipMemcpyAsync(spCount_.get(), &totalP_, sizeof(int64_t), hipMemcpyHostToDevice, st_), "spatial");
+    const SpatialBuild<T> b{es.P, es.stride, es.index, dSegs_.get(), ns, spItems_.get(), (int)items.size(),
+                            spFirst_.get(), spPartial_.get(), spMaps_.get(), bits, labS_.get()};
     check(launch_spatial_keys<T>(b, dim_, st_), "spatial keys");
-    check(stable_sort_by_key(labS_.get(), nullptr, dCount.get(), totalP_, numKeys, keys_.get(), spPerm_.get(),
+    check(stable_sort_by_key(labS_.get(), nullptr, spCount_.get(), totalP_, numKeys, keys_.get(), spPerm_.get(),
                              dM_.get(), sortWs_.get(), st_),
           "spatial sort");
     check(launch_spatial_gather<T>(es.P, es.stride, es.index, spPerm_.get(), totalP_, dim_, spQ_.get(), spStride_, st_),
@@ -1085,7 +1080,7 @@ void Engine<T>::buildSpatial() {
     check(launch_spatial_boxes<T>(spQ_.get(), spStride_, dBoxItems_.get(), dSegs_.get(), (int)boxItems_.size(), dim_,
                                   spBox_.get(), st_),
           "spatial boxes");
-    check(hipStreamSynchronize(st_), "spatial");   // the build's buffers are released on return
+    check(hipStreamSynchronize(st_), "spatial");   // the host vectors are released on return
     spatialValid_ = true;
 }
 
@@ -1608,18 +1603,16 @@ int Engine<T>::evolveIteration(int* labels, int* counts, T* sums, unsigned short
         check(hipMemcpyAsync(labels, labels_.get(), sizeof(int) * nPoints_, hipMemcpyDeviceToHost, st_), "labels");
     if (counts && total > 0)
         check(hipMemcpyAsync(counts, counts_.get(), sizeof(int) * total, hipMemcpyDeviceToHost, st_), "counts");
-    DevBuf<T> rows;
-    DevBuf<int64_t> dOff;
     std::vector<int64_t> off(ns, 0);
     if (sums && total > 0) {
         for (int s = 1; s < ns; ++s) off[s] = off[s - 1] + K[s - 1];
-        dOff.reserve(ns);
-        check(hipMemcpyAsync(dOff.get(), off.data(), sizeof(int64_t) * ns, hipMemcpyHostToDevice, st_), "off");
-        rows.reserve((size_t)total * dim_);
+        iterOff_.reserve(ns);
+        check(hipMemcpyAsync(iterOff_.get(), off.data(), sizeof(int64_t) * ns, hipMemcpyHostToDevice, st_), "off");
+        iterRows_.reserve((size_t)total * dim_);
         hipLaunchKernelGGL((gather_chosen_kernel<T>), dim3(ns), dim3(256), 0, st_, sums_.get(), sStride_, dSegs_.get(),
-                           dSegK_.get(), dOff.get(), dim_, rows.get(), (int)LAYOUT_ROW_MAJOR, (int64_t)dim_);
+                           dSegK_.get(), iterOff_.get(), dim_, iterRows_.get(), (int)LAYOUT_ROW_MAJOR, (int64_t)dim_);
         check(hipGetLastError(), "sums");
-        check(hipMemcpyAsync(sums, rows.get(), sizeof(T) * total * dim_, hipMemcpyDeviceToHost, st_), "sums");
+        check(hipMemcpyAsync(sums, iterRows_.get(), sizeof(T) * total * dim_, hipMemcpyDeviceToHost, st_), "sums");
     }
     std::vector<unsigned char> mv;
     if (moved && total > 0) {

@@ -295,6 +295,12 @@ private:
     int64_t spStride_ = 0;
     DevBuf<int> spPerm_, labS_, touched_, act_, movedSlot_, chainPrefix_;
     DevBuf<WorkItem> dBoxItems_;
+    // the build of the order (kept: freeing device memory makes every stream of the device wait)
+    DevBuf<WorkItem> spItems_;
+    DevBuf<int> spFirst_;
+    DevBuf<T> spPartial_;
+    DevBuf<SpatialMap<T>> spMaps_;
+    DevBuf<int64_t> spCount_;
     std::vector<WorkItem> boxItems_;
     void buildSpatial();
     bool prepareIncremental(long long iters);
@@ -328,6 +334,8 @@ private:
     DevBuf<unsigned char> sortWs_;
     DevBuf<int64_t> dN_, dM_;
     DevBuf<int> flags_;   // [0] allDone, [1] totalIters, [2] overflow
+    DevBuf<T> iterRows_;             // evolveIteration: sums as rows for the host
+    DevBuf<int64_t> iterOff_;
     // choose scratch
     DevBuf<int> chooseInfo_;         // choose: large segments, their filter blocks and state
     DevBuf<uint64_t> chooseOpen_;    // choose: samples of the large segments not decided yet
