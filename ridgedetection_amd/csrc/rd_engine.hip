@@ -1025,18 +1025,88 @@ void Engine<T>::autotuneBatchScan() {
     timers.tuneMs += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
+// Bits of the spatial key below the segment number.
+template <typename T>
+int Engine<T>::spatialBits() const {
+    int segBits = 0;
+    while ((int64_t(1) << segBits) < (int64_t)segs_.size()) ++segBits;
+    int maxP = 1;
+    for (const SegDesc& sd : segs_) maxP = std::max(maxP, (int)sd.nP);
+    // about 64 samples a cell of the largest segment (the occupied cells hold several times that)
+    return std::max(4, std::min({kSpatialBitsMax, ilog2(maxP) - 4, 30 - segBits}));
+}
+
+// Every buffer that incremental iterations over items of itemSize samples need beyond those of full
+// ones.  Where the device has no room for them, none is kept and the iterations are full ones: a cloud
+// whose full iterations fit must not fail for a second copy of its samples.
+template <typename T>
+bool Engine<T>::reserveIncremental(int itemSize) {
+    const size_t ns = segs_.size();
+    size_t bounds = 1, boxes = 1, items = 0;
+    for (const SegDesc& sd : segs_) {
+        bounds += (sd.nP + kBoundsItem - 1) / kBoundsItem;
+        boxes += (sd.nP + kBoxSamples - 1) / kBoxSamples;
+        items += (sd.nP + itemSize - 1) / itemSize;
+    }
+    const size_t slots = (size_t)std::max<int64_t>(totalSlots_, 1);
+    spStride_ = round_up(totalP_, 64);
+    try {
+        spItems_.reserve(bounds);
+        spFirst_.reserve(ns + 1);
+        spPartial_.reserve(bounds * 2 * dim_);
+        spMaps_.reserve(ns);
+        spCount_.reserve(1);
+        spQ_.reserve((size_t)spStride_ * dim_);
+        spPerm_.reserve(totalP_);
+        labS_.reserve(totalP_);
+        spBox_.reserve(boxes * 2 * dim_);
+        spBound_.reserve(boxes);
+        dBoxItems_.reserve(boxes);
+        touched_.reserve(slots);
+        act_.reserve(slots);
+        movedSlot_.reserve(slots);
+        Sold_.reserve((size_t)std::max<int64_t>(sStride_, 1) * dim_);
+        chainPrefix_.reserve((size_t)chainTable_);
+        sortWs_.reserve(sort_workspace_bytes(totalP_, (int)ns << spatialBits()));
+        // a growing buffer loses its items: the caller writes them anew for another item size
+        if (itemsPer_ != itemSize) dItems_.reserve(items);
+        return true;
+    } catch (const HipError& err) {
+        if (err.code != hipErrorOutOfMemory) throw;
+    }
+    (void)hipGetLastError();   // (the next launch check would report it)
+    spatialValid_ = false;
+    spItems_.release();
+    spFirst_.release();
+    spPartial_.release();
+    spMaps_.release();
+    spCount_.release();
+    spQ_.release();
+    spPerm_.release();
+    labS_.release();
+    spBox_.release();
+    spBound_.release();
+    dBoxItems_.release();
+    touched_.release();
+    act_.release();
+    movedSlot_.release();
+    Sold_.release();
+    chainPrefix_.release();
+    // full iterations use these two as well, and a buffer that could not grow is gone
+    ensureEvolveScratch();
+    buildWorkItems();
+    if (ns > 1) orderItemsByCost();
+    check(hipStreamSynchronize(st_), "full iterations");
+    return false;
+}
+
 // Spatial order of every segment's samples, their blocks and boxes (rd_spatial.hip).
 template <typename T>
 void Engine<T>::buildSpatial() {
     if (spatialValid_) return;
     const int ns = (int)segs_.size();
     const EvolveSource es = evolveSource();
-    int segBits = 0;
-    while ((int64_t(1) << segBits) < ns) ++segBits;
-    int maxP = 1;
-    for (const SegDesc& sd : segs_) maxP = std::max(maxP, (int)sd.nP);
-    // about 64 samples a cell of the largest segment (the occupied cells hold several times that)
-    const int bits = std::max(4, std::min({kSpatialBitsMax, ilog2(maxP) - 4, 30 - segBits}));
+    const int bits = spatialBits();
     std::vector<WorkItem> items;
     std::vector<int> firstItem(ns + 1);
     boxItems_.clear();
@@ -1049,19 +1119,6 @@ void Engine<T>::buildSpatial() {
     }
     firstItem[ns] = (int)items.size();
     const int numKeys = ns << bits;
-    spItems_.reserve(std::max<size_t>(items.size(), 1));
-    spFirst_.reserve(firstItem.size());
-    spPartial_.reserve(std::max<size_t>(items.size(), 1) * 2 * dim_);
-    spMaps_.reserve(ns);
-    spCount_.reserve(1);
-    spStride_ = round_up(totalP_, 64);
-    spQ_.reserve((size_t)spStride_ * dim_);
-    spPerm_.reserve(totalP_);
-    labS_.reserve(totalP_);
-    spBox_.reserve(std::max<size_t>(boxItems_.size(), 1) * 2 * dim_);
-    spBound_.reserve(std::max<size_t>(boxItems_.size(), 1));
-    dBoxItems_.reserve(std::max<size_t>(boxItems_.size(), 1));
-    sortWs_.reserve(sort_workspace_bytes(totalP_, numKeys));
     check(hipMemcpyAsync(spItems_.get(), items.data(), sizeof(WorkItem) * items.size(), hipMemcpyHostToDevice, st_), "sp");
     check(hipMemcpyAsync(spFirst_.get(), firstItem.data(), sizeof(int) * firstItem.size(), hipMemcpyHostToDevice, st_),
           "spatial");
@@ -1107,6 +1164,8 @@ bool Engine<T>::prepareIncremental(long long iters) {
     // scatter blocks: about one per CU or more, and no fewer samples than keys
     int itemSize = totalP_ < 131072 ? 256 : totalP_ < 262144 ? 512 : 1024;
     while (itemSize < 2048 && chainMeanKeys_ > itemSize) itemSize *= 2;
+    if (!chain_iteration_supported(dim_, itemSize, chainKeyCapMax_) || chainMeanKeys_ > itemSize) return false;
+    if (!reserveIncremental(itemSize)) return false;
     options.ppt = itemSize >= 1024 ? itemSize / 512 : itemSize / 256;
     options.scanThreads = itemSize >= 1024 ? 512 : 256;
     options.persistent = false;
@@ -1116,12 +1175,6 @@ bool Engine<T>::prepareIncremental(long long iters) {
     }
     if (!chainUsable(itemSize)) return false;
     buildSpatial();
-    const size_t slots = (size_t)std::max<int64_t>(totalSlots_, 1);
-    touched_.reserve(slots);
-    act_.reserve(slots);
-    movedSlot_.reserve(slots);
-    Sold_.reserve((size_t)std::max<int64_t>(sStride_, 1) * dim_);
-    chainPrefix_.reserve((size_t)chainTable_);
     if (!compact())   // (a batch uploads its active boxes)
         check(hipMemcpyAsync(dBoxItems_.get(), boxItems_.data(), sizeof(WorkItem) * boxItems_.size(),
                              hipMemcpyHostToDevice, st_),

@@ -302,6 +302,8 @@ private:
     DevBuf<SpatialMap<T>> spMaps_;
     DevBuf<int64_t> spCount_;
     std::vector<WorkItem> boxItems_;
+    int spatialBits() const;
+    bool reserveIncremental(int itemSize);
     void buildSpatial();
     bool prepareIncremental(long long iters);
     // expanded-form screen: table rows (dim + 1) x sStride_ and per-segment centre and bound
