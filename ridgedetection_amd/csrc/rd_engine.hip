@@ -115,9 +115,10 @@ inline unsigned grid_for(int64_t n) { return (unsigned)std::max<int64_t>(1, std:
 // the state of an evolve call for the host (Engine::polled_)
 __global__ void publish_kernel(const int* __restrict__ flags, const int* __restrict__ segDone, int numSegs,
                                int* __restrict__ out) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < 2) out[i] = flags[i];
-    if (i < numSegs) out[2 + i] = segDone[i];
+    const int first = blockIdx.x * 256 + threadIdx.x;
+    if (first < 2) out[first] = flags[first];
+    // (grid_for ends at 16,384 blocks)
+    for (int i = first; i < numSegs; i += (int)gridDim.x * 256) out[2 + i] = segDone[i];
 }
 
 // copies every segment's first `cnt` slots (coordinates and chosen indices) to a new layout
