@@ -95,8 +95,11 @@ typedef struct rdhip_timers {
     int64_t scan_ppt;        /* evolve scan shape in use: samples per lane ... */
     int64_t scan_threads;    /* ... and threads per block (after autotuning) */
     double tune_ms;          /* time spent timing candidate scan shapes */
-    double evolve_pairs;     /* (sample, chosen point) pairs the evolve iterations evaluated:
-                                per segment and iteration, its samples x its chosen points */
+    double evolve_pairs;     /* (sample, chosen point) pairs the evolve iterations decided: per
+                                segment and iteration, its samples x its chosen points.  Full scans
+                                evaluate all of them; incremental and segment-local iterations decide
+                                most by exact bounds or from the last iteration (evolve_bytes
+                                likewise counts what full iterations need) */
     int64_t scan_persistent; /* 1: the scan's blocks pull work items from a device queue */
     int64_t vjp_checkpoint_every;  /* iterations per recorded run of the last rdhip_evolve_fwd */
     int64_t chain_path;      /* 1: the last evolve iteration enqueued ordered its members with the
@@ -134,8 +137,9 @@ enum rdhip_option {
                                       (samples per lane x threads x persistent queue or not)
                                       shapes.  Cached per process.  Iterations that run
                                       incrementally (default options, at most 2048 and on average
-                                      at least 8 chosen points per segment) are not tuned; 0 keeps
-                                      every iteration a full scan */
+                                      at least 8 chosen points per segment, and device
+                                      memory for a second copy of the samples) are not tuned; 0
+                                      keeps every iteration a full scan */
     RDHIP_OPT_SEGMENTED = 10,      /* 1: a batch whose active segments all have at most 65536
                                       samples and 1024 chosen points iterates as a batch-wide scan
                                       plus one workgroup per segment for the member sort, ordered

@@ -22,9 +22,9 @@
 // total than one evolve scan; resolve is a dependence chain of ~40 cycles per chosen point.  The
 // form this replaces decided one survivor per block-wide barrier (~200 us per 256 samples that are
 // mostly chosen) and walked every 256 samples of a large cloud with one block (~0.7 us each, also
-// when all were covered).  Choose phase before -> after: 200k 6-D points with ~12,000 chosen
-// 173 -> 3.1 ms (13 resolves of 0.12 ms, 12 filters of 0.115 ms); 1M helix 6.2 -> 0.37 ms; 20k
-// spiral 1.49 -> 0.27 ms (5 resolves of 12 us); 2k spiral, one block, 241 -> 53 us.
+// when all were covered).  Choose phase before -> after: 200k 6-D points with ~11,000 chosen
+// 173 -> 3.1 ms (13 resolves of 0.12 ms, 12 filters of 0.118 ms); 1M helix 6.2 -> 0.27 ms (filters
+// of 21 us); 20k spiral 1.49 -> 0.14 ms (5 resolves of 12 us); 2k spiral, one block, 241 -> 53 us.
 #include "rd_choose.hpp"
 
 namespace rdhip {

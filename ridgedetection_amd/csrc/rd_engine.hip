@@ -757,12 +757,12 @@ void Engine<T>::enqueueIteration(bool record, int slot, const IterLog* log, bool
                                         chainSegHistOff_.get(), itemSize, flags_.get(), st_),
                       "label_hist");
         } else {
-        ScanArgs<T> sa{es.P, es.stride, es.index, S_.get(), sStride_, dItems_.get(), dSegs_.get(), dSegK_.get(),
-                       dSegDone_.get(), dSegR1Sqr_.get(), flags_.get(), labels, flags_.get() + 3,
-                       nullptr, nullptr, compact() ? flags_.get() + 4 : nullptr, nullptr, chainHist_.get(),
-                       chainSegHistOff_.get(), chainSegKeyCap_.get(), itemSize};
-        prepScreen(sa, screenForm());
-        check(launch_evolve_scan<T>(sa, dim_, itemsInUse(), options.ppt, options.scanThreads, 0, st_), "evolve_scan");
+            ScanArgs<T> sa{es.P, es.stride, es.index, S_.get(), sStride_, dItems_.get(), dSegs_.get(), dSegK_.get(),
+                           dSegDone_.get(), dSegR1Sqr_.get(), flags_.get(), labels, flags_.get() + 3,
+                           nullptr, nullptr, compact() ? flags_.get() + 4 : nullptr, nullptr, chainHist_.get(),
+                           chainSegHistOff_.get(), chainSegKeyCap_.get(), itemSize};
+            prepScreen(sa, screenForm());
+            check(launch_evolve_scan<T>(sa, dim_, itemsInUse(), options.ppt, options.scanThreads, 0, st_), "evolve_scan");
         }
         if (ev) check(hipEventRecord(events_[3 * slot + 1], st_), "event");
         enqueueChainOrder(itemSize, labels, inc, pending, capIter);
